@@ -95,13 +95,13 @@ __device__ __forceinline__ void runs_to_lds(const RowRuns& R, const T* __restric
 template <int RU>
 struct RunsAhead {
     int q0, q1;
-    int geo[RU], gm[RU];
+    int geo[RU];
     __device__ __forceinline__ void fetch(const RowRuns& R, int qb, int nt)
     {
 #pragma unroll
         for (int u = 0; u < RU; u++) {
             const int q = qb + u * nt;
-            if (q < q1) { geo[u] = R.geo[q]; gm[u] = R.gm[q]; }
+            if (q < q1) geo[u] = R.geo[q];
         }
     }
     __device__ __forceinline__ void prefetch(const RowRuns& R, int k, int ny, int y0, int nrows)
@@ -143,7 +143,7 @@ __device__ __forceinline__ void lds_to_runs(const RowRuns& R, RunsAhead<RU>& A, 
 #pragma unroll
                     for (int j = 0; j < MRMG_UF; j++) s += (double)(t + j < len ? a[j] : (T)0);
                 }
-                Hr[(size_t)(c0 + ci) * R.nruns + A.gm[u]] = s;
+                Hr[(size_t)(c0 + ci) * R.nruns + q] = s;
             }
         }
     }

@@ -285,9 +285,9 @@ struct Engine : EngineBase {
     std::vector<int> off;
     // grain data
     DBuf<int> layer_of, gc_off, cell2grain;
-    // runs (RowRuns): grain by grain (run_off per grain, run_geo, run_row) and row by row
-    // (rrow_off per layer row, rrm_geo, rrm_grain, rrm_gm)
-    DBuf<int> run_off, run_geo, run_row, rrow_off, rrm_geo, rrm_grain, rrm_gm;
+    // runs (RowRuns): grain by grain (run_off per grain, run_geo, run_row, run_q) and row by
+    // row (rrow_off per layer row, rrm_geo, rrm_grain)
+    DBuf<int> run_off, run_geo, run_row, run_q, rrow_off, rrm_geo, rrm_grain;
     int nruns = 0;
     DBuf<int> x_off, x_nb;
     DBuf<S> x_w;
@@ -304,7 +304,8 @@ struct Engine : EngineBase {
     DBuf<double> src_pos, src_vals, ax_xa, ax_xc, ax_ya, ax_yb, tlast;
     bool any_sg = false;   // a super-Gaussian temperature source on some layer
     DBuf<int> ax_xi, ax_yi;
-    bool any_src = false;
+    bool any_src = false, any_fsrc = false, all_sg = false;   // any moving source; field tables; only SG temperatures
+    int n_temp = 0;   // GrainData::n_temp
     // demag
     DBuf<C2<T>> S1, S2, Tspec, twx, twy;
     // Mg: the cell value Ms ms_scale m of every grain, [3][G]; Hr: the cell field summed
@@ -317,6 +318,7 @@ struct Engine : EngineBase {
     // launch shapes (mrmg_tune): threads of the row and column workgroups, observation-layer
     // groups per column workgroup, lanes per grain in the grain kernels
     int row_threads = 128, col_threads = 512, kg = 1, lpg = 8;
+    bool lpg_set = false;   // lanes_per_grain was tuned: build() leaves it
     // split column path (column-contiguous spectra): rows per row workgroup, columns per
     // column workgroup, and whether it is in use (forced by col_path or by the grid size)
     bool split = false, fused_ok = false, split_ok = false;
@@ -399,7 +401,7 @@ struct Engine : EngineBase {
         size_t b = 0;
         b += layer_of.bytes() + gc_off.bytes() + cell2grain.bytes();
         b += run_off.bytes() + run_geo.bytes() + run_row.bytes() + rrow_off.bytes() + rrm_geo.bytes() + rrm_grain.bytes() +
-             rrm_gm.bytes() + Mg.bytes() + Hr.bytes();
+             run_q.bytes() + Mg.bytes() + Hr.bytes();
         b += x_off.bytes() + x_nb.bytes() + x_w.bytes();
         b += ms.bytes() + msf.bytes() + ms_scale.bytes() + alpha_scale.bytes() + hk_scale.bytes() + hk1.bytes() +
              hk2.bytes() + uni.bytes() + cub.bytes() + happ.bytes() + sigma.bytes() + sigma_llb.bytes() + vol.bytes() +
@@ -549,6 +551,7 @@ struct Engine : EngineBase {
             if (v != 1 && v != 2 && v != 4 && v != 8 && v != 16)
                 return set_err(MRMG_ERR_ARG, "lanes_per_grain must be 1, 2, 4, 8 or 16");
             lpg = v;
+            lpg_set = true;
         } else if (k == "col_path") {
             if (v < 0 || v > 3)
                 return set_err(MRMG_ERR_ARG, "col_path must be 0 (fused), 1 (split), 2 (fused, column-contiguous) or 3 "
@@ -632,6 +635,11 @@ struct Engine : EngineBase {
         off.assign(nl + 1, 0);
         for (int k = 0; k < nl; k++) off[k + 1] = off[k] + L[k].ng;
         G = off[nl];
+        // one lane per grain where 64 grains a wave fill the chip (256 CUs of 4 SIMDs, two
+        // waves each), else as many lanes as keep the waves of the chip busy; measured, us a
+        // stage: 523 704 grains 161 with 1 lane, 195 with 2, 253 with 4; 32 680 grains 34, 26,
+        // 23; 15 692 grains 15.9, 13.0, 11.0 and 10.7 with 8
+        if (!lpg_set) lpg = G >= 131072 ? 1 : G >= 24576 ? 4 : 8;
         Ctot = 0;
         for (int k = 0; k < nl; k++) Ctot += L[k].ncell;
         std::vector<int> h_layer(G), h_gco(G + 1), h_gci(Ctot), h_c2g(nl * P, -1);
@@ -805,7 +813,7 @@ struct Engine : EngineBase {
                 rowoff[(size_t)layer[g] * ny + row[r] + 1]++;
             }
         for (size_t i = 1; i < rowoff.size(); i++) rowoff[i] += rowoff[i - 1];
-        std::vector<int> cur(rowoff.begin(), rowoff.end() - 1), rgeo(nruns), rgrain(nruns), rgm(nruns);
+        std::vector<int> cur(rowoff.begin(), rowoff.end() - 1), rgeo(nruns), rgrain(nruns), rq(nruns);
         std::vector<char> seen((size_t)nl * P, 0);
         for (int r = 0; r < nruns; r++) {
             const int g = grain_of[r];
@@ -819,18 +827,19 @@ struct Engine : EngineBase {
             const int q = cur[rw]++;
             rgeo[q] = geo[r];
             rgrain[q] = g;
-            rgm[q] = r;
+            rq[r] = q;
+            row[r] |= layer[g] << RUN_LAYER_SHIFT;
         }
         geo.push_back(0);   // no array is empty
         row.push_back(0);
-        rgeo.push_back(0); rgrain.push_back(0); rgm.push_back(0);
+        rgeo.push_back(0); rgrain.push_back(0); rq.push_back(0);
         RCHK(run_off.upload(roff.data(), roff.size(), c->stream));
         RCHK(run_geo.upload(geo.data(), geo.size(), c->stream));
         RCHK(run_row.upload(row.data(), row.size(), c->stream));
         RCHK(rrow_off.upload(rowoff.data(), rowoff.size(), c->stream));
         RCHK(rrm_geo.upload(rgeo.data(), rgeo.size(), c->stream));
         RCHK(rrm_grain.upload(rgrain.data(), rgrain.size(), c->stream));
-        RCHK(rrm_gm.upload(rgm.data(), rgm.size(), c->stream));
+        RCHK(run_q.upload(rq.data(), rq.size(), c->stream));
         HIPCHK(hipStreamSynchronize(c->stream));   // the host vectors go out of scope
         return MRMG_OK;
     }
@@ -838,7 +847,7 @@ struct Engine : EngineBase {
     RowRuns runs() const
     {
         RowRuns R;
-        R.row_off = rrow_off.p; R.geo = rrm_geo.p; R.grain = rrm_grain.p; R.gm = rrm_gm.p; R.nruns = nruns;
+        R.row_off = rrow_off.p; R.geo = rrm_geo.p; R.grain = rrm_grain.p; R.nruns = nruns;
         return R;
     }
 
@@ -847,7 +856,9 @@ struct Engine : EngineBase {
     {
         const int nl = c->nl, nx = c->nx, ny = c->ny;
         std::vector<double> pos, vals;
-        any_src = false;
+        any_src = any_fsrc = false;
+        n_temp = 0;
+        all_sg = true;
         for (int k = 0; k < nl; k++) {
             for (int sl = 0; sl < 2; sl++) {
                 SrcParams& sp = hlp[k].src[sl];
@@ -856,6 +867,14 @@ struct Engine : EngineBase {
                 sp.kind = q.kind;
                 if (q.kind == MRMG_SRC_NONE) continue;
                 any_src = true;
+                if (sl == 0) any_fsrc = true;
+                else {
+                    // an Ms that follows the temperature is taken at the next evaluation's
+                    const LayerParams& q0 = hlp[k];
+                    const bool dyn_ms = q0.tscale && !q0.use_mag && (q0.msexp >= 0.0 || q0.tab_n[0] > 1);
+                    n_temp = std::max(n_temp, dyn_ms ? 2 : 1);
+                    if (q.kind != MRMG_SRC_TEMP_SG) all_sg = false;
+                }
                 sp.nxp = q.nxp; sp.nyp = q.nyp; sp.expn = q.expn;
                 sp.vel_x = q.vel_x; sp.vel_y = q.vel_y; sp.offset_x = q.offset_x; sp.offset_y = q.offset_y;
                 sp.ref_x = q.ref_x; sp.ref_y = q.ref_y; sp.t_origin = q.t_origin; sp.isigx = q.isigx; sp.isigy = q.isigy;
@@ -976,13 +995,14 @@ struct Engine : EngineBase {
         d.ms = ms.p; d.msf = msf.p; d.ms_scale = ms_scale.p; d.alpha_scale = alpha_scale.p; d.hk_scale = hk_scale.p;
         d.hk1 = hk1.p; d.hk2 = hk2.p; d.uni = uni.p; d.cub = cub.p; d.happ = has_happ ? happ.p : nullptr;
         d.sigma = sigma.p; d.vol = vol.p; d.gc_off = gc_off.p;
-        d.run_off = run_off.p; d.run_geo = run_geo.p; d.run_row = run_row.p; d.nruns = nruns;
+        d.run_off = run_off.p; d.run_geo = run_geo.p; d.run_row = run_row.p; d.run_q = run_q.p; d.nruns = nruns;
         d.x_off = x_off.p; d.x_nb = x_nb.p; d.x_w = x_w.p;
         d.nl = c->nl;
         d.lp = lp.p;
         d.tc = tc.p; d.lam = lam.p; d.temp = temp.p; d.tabs = tabs.p;
         if (cur_llb) d.sigma = sigma_llb.p;
-        d.any_src = any_src;
+        d.any_fsrc = any_fsrc; d.n_temp = n_temp; d.all_sg = all_sg;
+        for (int k = 0; k <= MRMG_MAX_LAYERS; k++) d.loff[k] = off[std::min(k, c->nl)];
         d.ax.xi = ax_xi.p; d.ax.xa = ax_xa.p; d.ax.xc = ax_xc.p; d.ax.yi = ax_yi.p; d.ax.ya = ax_ya.p;
         d.ax.yb = ax_yb.p;
         d.ax.pos = src_pos.p; d.ax.vals = src_vals.p; d.ax.nx = c->nx; d.ax.ny = c->ny;
@@ -1118,7 +1138,7 @@ struct Engine : EngineBase {
     template <int MB> void launch_col_gen(int nb8);
     template <int MB> void launch_row_inv(dim3 g, dim3 b);
 
-    template <int MODE, int LPG> void launch_grain(const StepArgs& a, S* mout);
+    template <int MODE, int LPG> int launch_grain(const StepArgs& a, S* mout);
     template <int MODE> int grain(const StepArgs& a, S* mout = nullptr, double t_next = 0.0);
 
     // per-layer reductions of the last diag-enabled grain launch

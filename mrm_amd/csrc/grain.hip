@@ -15,9 +15,7 @@ __global__ void k_philox_dump(unsigned long long seed, unsigned long long step0,
 }
 
 // ------------------------------------------------------------------------- grain kernel
-// LPG lanes cooperate on one grain: the cell gather and the exchange sums are split over
-// the lanes and reduced with a fixed xor-butterfly (deterministic); the rest of the grain
-// work is computed redundantly by every lane and written by lane 0.
+// sum over the LPG lanes of a grain, a fixed xor-butterfly (deterministic)
 template <int LPG, typename T>
 __device__ __forceinline__ T lane_sum(T v)
 {
@@ -26,37 +24,13 @@ __device__ __forceinline__ T lane_sum(T v)
     return v;
 }
 
-// neighbour terms hx(j) ms_scale(nb) m(nb) of entries [j0, j1); the Ms scale is the
-// state's row ST_MSC.  Each lane takes entries j0+lane, j0+lane+LPG, ... in order; two
-// per round, with all index and value loads of a round issued before they are used.
-template <typename T, int LPG>
-__device__ __forceinline__ void csr_sum(int j0, int j1, const int* __restrict__ nb_, const T* __restrict__ w_,
-                                        const T* __restrict__ mf, int G, int lane, T* h)
+// element i of a uniform base: the byte offset in 32 bits (no array of the grain kernel has
+// 2^29 entries), so that a load takes one offset register per index, shared by the
+// component rows, instead of a 64-bit address each
+template <typename V>
+__device__ __forceinline__ V at32(const V* __restrict__ p, int i)
 {
-    T s0 = 0, s1 = 0, s2 = 0;
-    const T* __restrict__ msc = mf + (size_t)ST_MSC * G;
-    for (int ja = j0 + lane; ja < j1; ja += 2 * LPG) {
-        const int jb = ja + LPG;
-        const bool hb = jb < j1;
-        const int na = nb_[ja], nbb = hb ? nb_[jb] : 0;
-        const T wa = w_[ja], wb = hb ? w_[jb] : (T)0;
-        const T ca = msc[na], cb = msc[nbb];
-        const T ax = mf[na], ay = mf[G + na], az = mf[2 * G + na];
-        const T bx = mf[nbb], by = mf[G + nbb], bz = mf[2 * G + nbb];
-        T w = wa * ca;
-        s0 += w * ax;
-        s1 += w * ay;
-        s2 += w * az;
-        if (hb) {
-            w = wb * cb;
-            s0 += w * bx;
-            s1 += w * by;
-            s2 += w * bz;
-        }
-    }
-    h[0] += lane_sum<LPG>(s0);
-    h[1] += lane_sum<LPG>(s1);
-    h[2] += lane_sum<LPG>(s2);
+    return *reinterpret_cast<const V*>(reinterpret_cast<const char*>(p) + (size_t)((unsigned)i * (unsigned)sizeof(V)));
 }
 
 // Value of a moving source at cell (i, j) of layer k from the stage's axis tables:
@@ -74,14 +48,49 @@ __device__ __forceinline__ double src_cell(const SrcAxes& ax, const SrcParams& s
            (1.0 - fx) * yfc * v[nv * a11 + comp];
 }
 
+// A table source of layer k summed over the run of cells i0 .. i0+len-1 in row j at time
+// ts: src_cell's terms (NV components), the row's y weights read once and the four nodes'
+// values again only where the node along x changes.
+template <int NV>
+__device__ __forceinline__ void table_run(const SrcAxes& ax, const SrcParams& sp, int k, int slot, int ts, int i0,
+                                          int len, int j, double* out)
+{
+    const size_t bx = ((size_t)(k * 2 + slot) * 2 + ts) * ax.nx, by = ((size_t)(k * 2 + slot) * 2 + ts) * ax.ny;
+    const int iy = ax.yi[by + j];
+    const double yf = ax.ya[by + j], yfc = ax.yb[by + j];
+    const double* __restrict__ v = ax.vals + sp.voff + (size_t)NV * sp.nxp * (iy - 1);
+    double n[4][NV];
+    int last = -1;
+#pragma unroll
+    for (int c = 0; c < NV; c++) out[c] = 0.0;
+    for (int i = i0; i < i0 + len; i++) {
+        const int ix = ax.xi[bx + i];
+        const double fx = ax.xa[bx + i];
+        if (ix != last) {
+            const double* a = v + (size_t)NV * (ix - 1);
+            const double* b = a + (size_t)NV * sp.nxp;
+#pragma unroll
+            for (int c = 0; c < NV; c++) {
+                n[0][c] = a[c];
+                n[1][c] = a[NV + c];
+                n[2][c] = b[c];
+                n[3][c] = b[NV + c];
+            }
+            last = ix;
+        }
+#pragma unroll
+        for (int c = 0; c < NV; c++)
+            out[c] += fx * yf * n[0][c] + (1.0 - fx) * yf * n[1][c] + fx * yfc * n[2][c] + (1.0 - fx) * yfc * n[3][c];
+    }
+}
+
 // The super-Gaussian temperature source (slot 1) of layer k summed over the run of cells
 // i0 .. i0+len-1 in row j at time ts: ya[j] times the run's share of the running sums of
 // xa (the cells' own values ya[j] xa[i], get_sg, applied.f90:1792-1811, added up).
 __device__ __forceinline__ double sg_run(const SrcAxes& ax, int k, int ts, int i0, int len, int j)
 {
-    const size_t b = (size_t)(k * 2 + 1) * 2 + ts;
-    const double* xc = ax.xc + b * (ax.nx + 1);
-    return ax.ya[b * ax.ny + j] * (xc[i0 + len] - xc[i0]);
+    const int b = (k * 2 + 1) * 2 + ts, x0 = b * (ax.nx + 1) + i0;
+    return at32(ax.ya, b * ax.ny + j) * (at32(ax.xc, x0 + len) - at32(ax.xc, x0));
 }
 
 // (1 - T/Tc)^e clamped to [0, 1] (temp_scaling.f90:390-395)
@@ -109,15 +118,9 @@ __device__ __forceinline__ double scale_at_t(const LayerParams& L, const double*
     return table_eval(tt, tt + L.tab_n[q], L.tab_n[q], T / Tc);
 }
 
-// tout (may be null): the grain temperature at the evaluation and at the next evaluation
-// from the layer's temperature source (field.f90:545-556); unchanged without one.
-// Loads are arranged for memory-level parallelism: the offsets and constants first, then
-// per round (each lane two cells and two exchange entries) all index loads, then all value
-// loads, then the sums.  Out-of-range positions load a valid entry (the arrays carry one
-// spare entry at the end) and add nothing.
-// Per-grain offsets and field constants, loaded by the caller with the grain's state.
+// Per-grain field constants.
 template <typename T> struct GrainPre {
-    int b0, b1, r0, r1, x0, x1;   // cell range (grain2gridindex: its count), run range, exchange CSR range
+    int cells;   // grain2gridindex: its cell count
     T hk_s, hk1, hk2, u[3], happ[3];
 };
 
@@ -125,9 +128,7 @@ template <typename T>
 __device__ __forceinline__ void grain_pre(const GrainData<T>& gd, int g, GrainPre<T>& P)
 {
     const int G = gd.G;
-    P.b0 = gd.gc_off[g]; P.b1 = gd.gc_off[g + 1];
-    P.r0 = gd.run_off[g]; P.r1 = gd.run_off[g + 1];
-    P.x0 = gd.x_off[g]; P.x1 = gd.x_off[g + 1];
+    P.cells = gd.gc_off[g + 1] - gd.gc_off[g];
     P.hk_s = gd.hk_scale[g]; P.hk1 = gd.hk1[g]; P.hk2 = gd.hk2[g];
     P.u[0] = gd.uni[g]; P.u[1] = gd.uni[G + g]; P.u[2] = gd.uni[2 * G + g];
     P.happ[0] = P.happ[1] = P.happ[2] = 0;
@@ -136,116 +137,328 @@ __device__ __forceinline__ void grain_pre(const GrainData<T>& gd, int g, GrainPr
     }
 }
 
-template <typename T, int LPG, typename TC>
-__device__ __forceinline__ void field_at(const GrainData<T>& gd, const LayerParams& L, int k, int g, int lane,
-                                         const T* __restrict__ mf, const double* __restrict__ Hr,
-                                         double t, const T* m, T* h, double* tout, GrainPre<T>& P)
+// The sums a grain's field is assembled from: the demag field of its runs, the exchange
+// terms, its runs' source temperature (n_temp: none, at the evaluation, or also at the next
+// one, which only an Ms that follows the temperature needs) and its runs' field table.
+struct GrainSums {
+    double hd[3], hx[3], t[2], hs[3];
+};
+
+// A wave takes 64 / LPG consecutive grains, whose runs and exchange entries are consecutive
+// too.  Its 64 lanes load them, a run and an entry per lane and slot and U slots a round,
+// all index loads of a round before its value loads, and leave the values in the wave's own
+// LDS; then a lane per grain adds up its grain's in their order.  The kernel is bound by the
+// latency of dependent loads (run -> its sum, entry -> neighbour -> its state), so what
+// counts is how many are in flight and how few cache lines each touches: consecutive lanes
+// read consecutive runs.  Waves do not wait for each other.  (With a loop over its runs in
+// each grain's own lanes, 8 lanes a grain, a stage of the 2048x2048x8 write took 497 / 487
+// us, and 200 us with one lane a grain.)
+template <int LPG> struct GrainShape {
+    static constexpr int U = 4;   // two, three: 178, 168 against 161 us in the 2048x2048x8 write
+    static constexpr int CH = 64 * U;
+    // an LDS slot of val: one spare every 8, so that grains of 8 entries do not share banks
+    static constexpr int SLOTS = CH + CH / 8;
+    // the channels in LDS at a time: the demag field and the temperatures, or a vector
+    static __host__ __device__ int doubles(int n_temp) { return SLOTS * (3 + n_temp); }
+};
+
+// the slots [a, b) of one channel added up in order
+__device__ __forceinline__ double slot_sum(const double* v, int a, int b, double s)
 {
-    const int G = gd.G;
-    const bool fsrc = L.src[0].kind == MRMG_SRC_FIELD_TABLE, tsrc = L.src[1].kind != MRMG_SRC_NONE;
-    const int b0 = P.b0, b1 = P.b1, x0 = P.x0, x1 = P.x1;
-    const T hk_s = P.hk_s, hk1 = P.hk1, hk2 = P.hk2;
-    const T u[3] = {P.u[0], P.u[1], P.u[2]};
-    T happ[3] = {P.happ[0], P.happ[1], P.happ[2]};
-    const T* __restrict__ msc = mf + (size_t)ST_MSC * G;
-    // get_magnetostatic gather (field.f90:463-468), summed over the grain's runs (each run
-    // the sum of its cells, written by the row c2r), and the exchange CSR
-    // (field.f90:326-363: intralayer, then the layers above and below, merged per grain)
-    const int r0 = P.r0, r1 = P.r1;
+    for (int j = a; j < b; j++) s += v[j + (j >> 3)];
+    return s;
+}
+
+// The sums of the wave's ngw grains from gw0 on, lane l holding those of grain gw0 + l (l <
+// ngw).  mf: the state the field is taken at; Hr: the run sums of the demag field, or null;
+// temps_only: the temperatures alone.  val: the wave's LDS.
+template <typename T, int LPG>
+__device__ __forceinline__ void grain_sums(const GrainData<T>& gd, const LayerParams* lp, int gw0, int ngw,
+                                           const T* __restrict__ mf, const double* __restrict__ Hr, bool temps_only,
+                                           double* val, GrainSums& S)
+{
+    typedef GrainShape<LPG> Sh;
+    constexpr int U = Sh::U, CH = Sh::CH, SL = Sh::SLOTS;
+    const int l = (int)threadIdx.x & 63, G = gd.G, nt = gd.n_temp;
+    const bool fsrc = gd.any_fsrc && !temps_only;
+    const int r0 = gd.run_off[gw0], r1 = gd.run_off[gw0 + ngw], x0 = gd.x_off[gw0], x1 = gd.x_off[gw0 + ngw];
+    const int gl = gw0 + (l < ngw ? l : 0);
+    const int ra = gd.run_off[gl] - r0, rb = gd.run_off[gl + 1] - r0;
+    const int xa = gd.x_off[gl] - x0, xb = gd.x_off[gl + 1] - x0;
     const size_t NR = (size_t)gd.nruns;
-    T hd[3] = {0, 0, 0}, hx[3] = {0, 0, 0};
-    double hs[3] = {0, 0, 0}, ts0 = 0, ts1 = 0;
-    if (!fsrc && !tsrc) {
-        T s0 = 0, s1 = 0, s2 = 0, e0 = 0, e1 = 0, e2 = 0;
-        const int nrun = r1 - r0, ne = x1 - x0;
-        const int ncr = (nrun + 2 * LPG - 1) / (2 * LPG), ner = (ne + 2 * LPG - 1) / (2 * LPG);
-        const int nr = ncr > ner ? ncr : ner;
-        for (int r = 0; r < nr; r++) {
-            const int qa = r0 + lane + 2 * r * LPG, qb = qa + LPG;
-            const int ja = x0 + lane + 2 * r * LPG, jb = ja + LPG;
-            const bool hqa = qa < r1, hqb = qb < r1, hja = ja < x1, hjb = jb < x1;
-            const int na = gd.x_nb[hja ? ja : x0], nbb = gd.x_nb[hjb ? jb : x0];
-            const T wa = gd.x_w[hja ? ja : x0], wb = gd.x_w[hjb ? jb : x0];
-            T c0 = 0, c1 = 0, c2 = 0, d0 = 0, d1 = 0, d2 = 0;
-            if (Hr) {
-                const int ra = hqa ? qa : r0, rb = hqb ? qb : r0;
-                c0 = (T)Hr[ra]; c1 = (T)Hr[NR + ra]; c2 = (T)Hr[2 * NR + ra];
-                d0 = (T)Hr[rb]; d1 = (T)Hr[NR + rb]; d2 = (T)Hr[2 * NR + rb];
-            }
-            const T pa = msc[na], pb = msc[nbb];
-            const T ax = mf[na], ay = mf[G + na], az = mf[2 * G + na];
-            const T bx = mf[nbb], by = mf[G + nbb], bz = mf[2 * G + nbb];
-            if (hqa) { s0 += c0; s1 += c1; s2 += c2; }
-            if (hqb) { s0 += d0; s1 += d1; s2 += d2; }
-            if (hja) {
-                const T w = wa * pa;
-                e0 += w * ax; e1 += w * ay; e2 += w * az;
-            }
-            if (hjb) {
-                const T w = wb * pb;
-                e0 += w * bx; e1 += w * by; e2 += w * bz;
-            }
-        }
-        if (Hr) {
-            const T cnt = (T)(b1 - b0);
-            hd[0] = lane_sum<LPG>(s0) / cnt;
-            hd[1] = lane_sum<LPG>(s1) / cnt;
-            hd[2] = lane_sum<LPG>(s2) / cnt;
-        }
-        hx[0] = lane_sum<LPG>(e0);
-        hx[1] = lane_sum<LPG>(e1);
-        hx[2] = lane_sum<LPG>(e2);
-    } else {
-        // moving sources: a table is sampled at every cell of the grain's runs; the
-        // separable super-Gaussian temperature is summed per run from its running sums
-        T s0 = 0, s1 = 0, s2 = 0;
-        const bool tsg = tsrc && L.src[1].kind == MRMG_SRC_TEMP_SG;
-        const bool per_cell = fsrc || (tsrc && !tsg);
-        for (int q = r0 + lane; q < r1; q += LPG) {
-            if (Hr) {
-                s0 += (T)Hr[q];
-                s1 += (T)Hr[NR + q];
-                s2 += (T)Hr[2 * NR + q];
-            }
-            const int geo = gd.run_geo[q], j = gd.run_row[q];
-            const int i0 = geo & 0xffff, len = geo >> 16;
-            if (tsg) {
-                ts0 += sg_run(gd.ax, k, 0, i0, len, j);
-                ts1 += sg_run(gd.ax, k, 1, i0, len, j);
-            }
-            if (per_cell)
-                for (int i = i0; i < i0 + len; i++) {
-                    if (fsrc)
+    const T* __restrict__ msc = mf + (size_t)ST_MSC * G;
 #pragma unroll
-                        for (int c = 0; c < 3; c++) hs[c] += src_cell(gd.ax, L.src[0], k, 0, 0, i, j, c, 3);
-                    if (tsrc && !tsg) {
-                        ts0 += src_cell(gd.ax, L.src[1], k, 1, 0, i, j, 0, 1);
-                        ts1 += src_cell(gd.ax, L.src[1], k, 1, 1, i, j, 0, 1);
+    for (int c = 0; c < 3; c++) S.hd[c] = S.hx[c] = S.hs[c] = 0.0;
+    S.t[0] = S.t[1] = 0.0;
+    const int nr = r1 - r0, nx = x1 - x0, n = temps_only || nr > nx ? nr : nx;
+    const bool src = nt > 0 || fsrc;
+    for (int cb = 0; cb < n; cb += CH) {
+        // positions past the end load a valid entry; their slots are never added
+        double xv[U][3];
+        int geo[U], row[U];
+        {
+            int q[U], nb[U];
+            double w[U], hv[U][3], xs[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int i = cb + l + 64 * u;
+                const int r = r0 + (i < nr ? i : 0), e = x0 + (i < nx ? i : 0);
+                if (!temps_only) {
+                    q[u] = at32(gd.run_q, r);
+                    nb[u] = at32(gd.x_nb, e);
+                    w[u] = at32(gd.x_w, e);
+                }
+                if (src) {
+                    geo[u] = at32(gd.run_geo, r);
+                    row[u] = at32(gd.run_row, r);
+                }
+            }
+            if (!temps_only) {
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+#pragma unroll
+                    for (int c = 0; c < 3; c++) {
+                        hv[u][c] = Hr ? at32(Hr + c * NR, q[u]) : 0.0;
+                        xv[u][c] = at32(mf + (size_t)c * G, nb[u]);
+                    }
+                    xs[u] = at32(msc, nb[u]);
+                }
+            }
+            if (nt > 0 && gd.all_sg) {
+                // a layer without a source reads tables that no kernel filled, and none of
+                // its grains uses the sum
+                double tv[U][2];
+#pragma unroll
+                for (int u = 0; u < U; u++)
+#pragma unroll
+                    for (int ts = 0; ts < 2; ts++)
+                        if (ts < nt)
+                            tv[u][ts] = sg_run(gd.ax, row[u] >> RUN_LAYER_SHIFT, ts, geo[u] & 0xffff, geo[u] >> 16,
+                                               row[u] & RUN_ROW_MASK);
+#pragma unroll
+                for (int u = 0; u < U; u++)
+#pragma unroll
+                    for (int ts = 0; ts < 2; ts++)
+                        if (ts < nt) val[(3 + ts) * SL + 72 * u + l + (l >> 3)] = tv[u][ts];
+            }
+            if (!temps_only) {
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const double wm = w[u] * xs[u];
+#pragma unroll
+                    for (int c = 0; c < 3; c++) {
+                        val[c * SL + 72 * u + l + (l >> 3)] = hv[u][c];
+                        xv[u][c] *= wm;
+                    }
+                }
+            }
+            if (nt > 0 && !gd.all_sg)
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    if (cb + l + 64 * u >= nr) break;
+                    const int i0 = geo[u] & 0xffff, len = geo[u] >> 16, k = row[u] >> RUN_LAYER_SHIFT,
+                              j = row[u] & RUN_ROW_MASK;
+                    for (int ts = 0; ts < nt; ts++) {
+                        const SrcParams& sp = lp[k].src[1];
+                        double v = 0.0;
+                        if (sp.kind == MRMG_SRC_TEMP_SG) v = sg_run(gd.ax, k, ts, i0, len, j);
+                        else if (sp.kind != MRMG_SRC_NONE) table_run<1>(gd.ax, sp, k, 1, ts, i0, len, j, &v);
+                        val[(3 + ts) * SL + 72 * u + l + (l >> 3)] = v;
                     }
                 }
         }
-        const T cnt = (T)(b1 - b0);
-        if (Hr) {
-            hd[0] = lane_sum<LPG>(s0) / cnt;
-            hd[1] = lane_sum<LPG>(s1) / cnt;
-            hd[2] = lane_sum<LPG>(s2) / cnt;
-        }
-        const double dc = (double)(b1 - b0);
-        if (fsrc)
+        wave_sync();
+        if (l < ngw) {
+            const int a = ra > cb ? ra - cb : 0, b = rb - cb < CH ? rb - cb : CH;
+            if (!temps_only)
 #pragma unroll
-            for (int c = 0; c < 3; c++) hs[c] = lane_sum<LPG>(hs[c]) / dc;
-        if (tsrc && tout) {
-            const double tst = gd.temp[g];
-            tout[0] = lane_sum<LPG>(ts0) / dc + tst;
-            tout[1] = lane_sum<LPG>(ts1) / dc + tst;
+                for (int c = 0; c < 3; c++) S.hd[c] = slot_sum(val + c * SL, a, b, S.hd[c]);
+            if (nt > 0) S.t[0] = slot_sum(val + 3 * SL, a, b, S.t[0]);
+            if (nt > 1) S.t[1] = slot_sum(val + 4 * SL, a, b, S.t[1]);
         }
-        csr_sum<T, LPG>(x0, x1, gd.x_nb, gd.x_w, mf, G, lane, hx);
+        wave_sync();
+        if (fsrc) {
+            // the field tables' sums through the same slots
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                if (cb + l + 64 * u >= nr) break;
+                const int k = row[u] >> RUN_LAYER_SHIFT;
+                double v[3] = {0.0, 0.0, 0.0};
+                if (lp[k].src[0].kind == MRMG_SRC_FIELD_TABLE)
+                    table_run<3>(gd.ax, lp[k].src[0], k, 0, 0, geo[u] & 0xffff, geo[u] >> 16, row[u] & RUN_ROW_MASK, v);
+#pragma unroll
+                for (int c = 0; c < 3; c++) val[c * SL + 72 * u + l + (l >> 3)] = v[c];
+            }
+            wave_sync();
+            if (l < ngw) {
+                const int a = ra > cb ? ra - cb : 0, b = rb - cb < CH ? rb - cb : CH;
+#pragma unroll
+                for (int c = 0; c < 3; c++) S.hs[c] = slot_sum(val + c * SL, a, b, S.hs[c]);
+            }
+            wave_sync();
+        }
+        if (!temps_only) {
+            // the exchange terms through the same slots
+#pragma unroll
+            for (int u = 0; u < U; u++)
+#pragma unroll
+                for (int c = 0; c < 3; c++) val[c * SL + 72 * u + l + (l >> 3)] = xv[u][c];
+            wave_sync();
+            if (l < ngw) {
+                const int a = xa > cb ? xa - cb : 0, b = xb - cb < CH ? xb - cb : CH;
+#pragma unroll
+                for (int c = 0; c < 3; c++) S.hx[c] = slot_sum(val + c * SL, a, b, S.hx[c]);
+            }
+            wave_sync();
+        }
+    }
+}
+
+// The sums of grain g by its own LPG lanes (4 and more lanes a grain, for media too small to
+// fill the chip with 64 grains a wave), which meet in a fixed butterfly: fewer steps one
+// after the other than through LDS (256x256x4, 15 692 grains, 8 lanes: 10.9 against 13.3 us).
+// LaneRound holds the index loads of a round, so that the first can be under way before the
+// workgroup's barrier.
+template <int LPG> struct LaneRound {
+    static constexpr int U = LPG <= 4 ? 2 : 1;   // runs and entries per lane and round
+    int r0, r1, x0, x1;
+    int q[U], nb[U], geo[U], row[U];
+    double w[U];
+    __device__ __forceinline__ void range(const int* run_off, const int* x_off, int g)
+    {
+        r0 = run_off[g]; r1 = run_off[g + 1];
+        x0 = x_off[g]; x1 = x_off[g + 1];
+    }
+    // positions past the end load a valid entry, which is not added
+    template <typename T> __device__ __forceinline__ void load(const GrainData<T>& gd, int b, bool src)
+    {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int r = r0 + b + u * LPG, e = x0 + b + u * LPG, rc = r < r1 ? r : r0, ec = e < x1 ? e : x0;
+            q[u] = at32(gd.run_q, rc);
+            nb[u] = at32(gd.x_nb, ec);
+            w[u] = at32(gd.x_w, ec);
+            if (src) {
+                geo[u] = at32(gd.run_geo, rc);
+                row[u] = at32(gd.run_row, rc);
+            }
+        }
+    }
+};
+
+template <typename T, int LPG>
+__device__ __forceinline__ void grain_sums_lanes(const GrainData<T>& gd, const LayerParams* lp, int k, int lane,
+                                                 const T* __restrict__ mf, const double* __restrict__ Hr,
+                                                 bool temps_only, LaneRound<LPG>& I, GrainSums& S)
+{
+    constexpr int U = LaneRound<LPG>::U;
+    const int G = gd.G, nt = gd.n_temp;
+    const bool fsrc = gd.any_fsrc && !temps_only && lp[k].src[0].kind == MRMG_SRC_FIELD_TABLE;
+    const bool tsrc = nt > 0 && lp[k].src[1].kind != MRMG_SRC_NONE;
+    const bool tsg = tsrc && lp[k].src[1].kind == MRMG_SRC_TEMP_SG;
+    const size_t NR = (size_t)gd.nruns;
+    const T* __restrict__ msc = mf + (size_t)ST_MSC * G;
+    double hd[3] = {0, 0, 0}, hx[3] = {0, 0, 0}, tt[2] = {0, 0}, hs[3] = {0, 0, 0};
+    const int nr = I.r1 - I.r0, nx = I.x1 - I.x0, n = temps_only || nr > nx ? nr : nx;
+    for (int b = lane; b < n; b += U * LPG) {
+        double hv[U][3], xv[U][4], tv[U][2];
+        if (!temps_only)
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+#pragma unroll
+                for (int c = 0; c < 3; c++) {
+                    hv[u][c] = Hr ? at32(Hr + c * NR, I.q[u]) : 0.0;
+                    xv[u][c] = at32(mf + (size_t)c * G, I.nb[u]);
+                }
+                xv[u][3] = at32(msc, I.nb[u]);
+            }
+        if (tsg)
+#pragma unroll
+            for (int u = 0; u < U; u++)
+#pragma unroll
+                for (int ts = 0; ts < 2; ts++)
+                    if (ts < nt)
+                        tv[u][ts] = sg_run(gd.ax, k, ts, I.geo[u] & 0xffff, I.geo[u] >> 16, I.row[u] & RUN_ROW_MASK);
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const bool hr = b + u * LPG < nr;
+            if (!temps_only) {
+                if (hr) {
+#pragma unroll
+                    for (int c = 0; c < 3; c++) hd[c] += hv[u][c];
+                }
+                if (b + u * LPG < nx) {
+                    const double wm = I.w[u] * xv[u][3];
+#pragma unroll
+                    for (int c = 0; c < 3; c++) hx[c] += wm * xv[u][c];
+                }
+            }
+            if (tsg && hr) {
+                tt[0] += tv[u][0];
+                if (nt > 1) tt[1] += tv[u][1];
+            }
+        }
+        if ((tsrc && !tsg) || fsrc)
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                if (b + u * LPG >= nr) break;
+                const int i0 = I.geo[u] & 0xffff, len = I.geo[u] >> 16, j = I.row[u] & RUN_ROW_MASK;
+                double v[3];
+                if (tsrc && !tsg)
+                    for (int ts = 0; ts < nt; ts++) {
+                        table_run<1>(gd.ax, lp[k].src[1], k, 1, ts, i0, len, j, v);
+                        tt[ts] += v[0];
+                    }
+                if (fsrc) {
+                    table_run<3>(gd.ax, lp[k].src[0], k, 0, 0, i0, len, j, v);
+#pragma unroll
+                    for (int c = 0; c < 3; c++) hs[c] += v[c];
+                }
+            }
+        if (b + U * LPG < n) I.load(gd, b + U * LPG, nt > 0 || gd.any_fsrc);
+    }
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+        S.hd[c] = lane_sum<LPG>(hd[c]);
+        S.hx[c] = lane_sum<LPG>(hx[c]);
+        S.hs[c] = fsrc ? lane_sum<LPG>(hs[c]) : 0.0;
+    }
+    S.t[0] = tsrc ? lane_sum<LPG>(tt[0]) : 0.0;
+    S.t[1] = tsrc && nt > 1 ? lane_sum<LPG>(tt[1]) : 0.0;
+}
+
+// the field of grain g from its sums; tout: the grain temperature at the
+// evaluation and at the next evaluation from the layer's temperature source
+// (field.f90:545-556), unchanged without one
+template <typename T>
+__device__ __forceinline__ void field_at(const GrainData<T>& gd, const LayerParams& L, int g, const GrainSums& S,
+                                         bool demag, double t, const T* m, T* h, double* tout, const GrainPre<T>& P)
+{
+    const int G = gd.G;
+    const bool fsrc = L.src[0].kind == MRMG_SRC_FIELD_TABLE, tsrc = L.src[1].kind != MRMG_SRC_NONE;
+    const T hk_s = P.hk_s, hk1 = P.hk1, hk2 = P.hk2;
+    const T u[3] = {P.u[0], P.u[1], P.u[2]};
+    T happ[3] = {P.happ[0], P.happ[1], P.happ[2]};
+    // get_magnetostatic gather (field.f90:463-468): the runs' sums (each run the sum of its
+    // cells, written by the row c2r) over the cell count; the exchange CSR
+    // (field.f90:326-363: intralayer, then the layers above and below, merged per grain)
+    const T cnt = (T)P.cells;
+    T hd[3] = {0, 0, 0}, hx[3];
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+        if (demag) hd[c] = S.hd[c] / cnt;
+        hx[c] = S.hx[c];
+    }
+    if (tsrc) {
+        const double tst = gd.temp[g];
+        tout[0] = S.t[0] / cnt + tst;
+        if (gd.n_temp > 1) tout[1] = S.t[1] / cnt + tst;
     }
     // get_applied: static per-grain field + source average + uniform ramped field
     // (applied.f90:871-883)
     if (fsrc)
 #pragma unroll
-        for (int i = 0; i < 3; i++) happ[i] = happ[i] + (T)hs[i];
+        for (int i = 0; i < 3; i++) happ[i] = happ[i] + S.hs[i] / cnt;
     if (L.has_uf) {
         const double sc = tscale_eval(L.uf_fn, L.uf_t0, L.uf_t1, L.uf_s0, L.uf_s1, L.uf_scale, t);
 #pragma unroll
@@ -255,7 +468,7 @@ __device__ __forceinline__ void field_at(const GrainData<T>& gd, const LayerPara
     for (int i = 0; i < 3; i++) h[i] = happ[i] + hd[i];
     // find_temp_scaling of Hk at the evaluation's temperature (temp_scaling.f90:392-395)
     T hks = hk_s;
-    if (tsrc && tout && scale_follows_t(L, 2)) hks = (T)scale_at_t(L, gd.tabs, 2, tout[0], gd.tc[g]);
+    if (tsrc && scale_follows_t(L, 2)) hks = (T)scale_at_t(L, gd.tabs, 2, tout[0], gd.tc[g]);
     // get_cubic_hk (field.f90:377-395)
     if (L.has_cub && hks > (T)0) {
         const T* A = gd.cub;
@@ -294,7 +507,7 @@ __device__ __forceinline__ void src_temp(const GrainData<T>& gd, const LayerPara
     double ts0 = 0, ts1 = 0;
     const bool tsg = L.src[1].kind == MRMG_SRC_TEMP_SG;
     for (int q = r0 + lane; q < r1; q += LPG) {
-        const int geo = gd.run_geo[q], j = gd.run_row[q];
+        const int geo = gd.run_geo[q], j = gd.run_row[q] & RUN_ROW_MASK;
         const int i0 = geo & 0xffff, len = geo >> 16;
         if (tsg) {
             ts0 += sg_run(gd.ax, k, 0, i0, len, j);
@@ -706,40 +919,64 @@ __global__ void __launch_bounds__(256) k_grain(GrainData<T> gd, T* __restrict__ 
     const int nblk = (gd.G * LPG + 255) / 256;
     const int bl = xcd_remap(blockIdx.x, gridDim.x);
     if (bl >= nblk) return;
-    const int tid = bl * blockDim.x + threadIdx.x;
     const int G = gd.G;
-    // threads past the last grain repeat the last grain's work and store nothing, so the
-    // loads below need no guard; every lane of a grain computes its results, lane 0 stores
-    const bool act = tid / LPG < G;
-    const int g = act ? tid / LPG : G - 1, lane = tid % LPG;
-    const bool w0 = act && lane == 0;
+    // LPG <= 2: lane l < 64 / LPG of a wave has the wave's grain l and the other lanes only
+    // help to load; else every lane of a grain computes its results and its first one stores
+    constexpr bool WAVE = LPG <= 2;
+    constexpr int NGW = 64 / LPG;
+    const int wv = (int)threadIdx.x >> 6, ln = (int)threadIdx.x & 63;
+    const int gw0 = __builtin_amdgcn_readfirstlane(bl * (256 / LPG) + wv * NGW);
+    const int ngw = G - gw0 < NGW ? G - gw0 : NGW;   // <= 0: this wave has none
+    const int gl = WAVE ? ln : ln / LPG;
+    const bool act = gl < ngw, w0 = WAVE || ln % LPG == 0;
+    const int g = act ? gw0 + gl : G - 1;
+    extern __shared__ __align__(16) double gval[];
     __shared__ double red[DIAG_STRIDE];
     __shared__ LayerParams slp[MRMG_MAX_LAYERS];
-    // the grain's state and constants, issued first; the layer parameters' copy into LDS
-    // then waits for all of them at once
     const int k = gd.layer_of[g];
-    GrainPre<T> P;
-    grain_pre(gd, g, P);
     const T* mf = (MODE == GM_HEUN2 || MODE == GM_ROT2) ? mb : ma;
-    T mfield[3] = {mf[g], mf[G + g], mf[2 * G + g]};
-    const T mi[3] = {ma[g], ma[G + g], ma[2 * G + g]};
-    const T msc = mf[(size_t)ST_MSC * G + g];
-    const T g_ms = gd.ms[g], g_msf = gd.msf[g], g_vol = gd.vol[g], g_sig = gd.sigma[g];
-    T g_as = gd.alpha_scale[g];
-    const double g_temp = gd.temp[g];
-    T dmv[3] = {0, 0, 0}, thv[3] = {0, 0, 0};
-    if (MODE == GM_HEUN2)
+    // the grain's state and constants: with 8 and more lanes a grain issued first, so that
+    // they overlap the sums' loads; with fewer loaded after the sums, since held across them
+    // they would cost waves in flight (250 registers against 162 with one lane, 264 against
+    // 154 with four: 30.9 against 22.0 us at 32 680 grains)
+    GrainPre<T> P;
+    T mfield[3], mi[3], msc, g_ms, g_msf, g_vol, g_sig, g_as, dmv[3] = {0, 0, 0}, thv[3] = {0, 0, 0};
+    double g_temp;
+    auto load = [&]() {
+        grain_pre(gd, g, P);
 #pragma unroll
-        for (int c = 0; c < 3; c++) dmv[c] = dm[(size_t)c * G + g];
-    if (!(MODE == GM_HEUN1 || MODE == GM_ROT1 || MODE == GM_FIELD1))
-#pragma unroll
-        for (int c = 0; c < 3; c++) thv[c] = hthm[(size_t)c * G + g];
+        for (int c = 0; c < 3; c++) {
+            mfield[c] = mf[(size_t)c * G + g];
+            mi[c] = ma[(size_t)c * G + g];
+            if (MODE == GM_HEUN2) dmv[c] = dm[(size_t)c * G + g];
+            if (!(MODE == GM_HEUN1 || MODE == GM_ROT1 || MODE == GM_FIELD1)) thv[c] = hthm[(size_t)c * G + g];
+        }
+        msc = mf[(size_t)ST_MSC * G + g];
+        g_ms = gd.ms[g]; g_msf = gd.msf[g]; g_vol = gd.vol[g]; g_sig = gd.sigma[g];
+        g_as = gd.alpha_scale[g];
+        g_temp = gd.temp[g];
+    };
+    LaneRound<WAVE ? 8 : LPG> I;
+    if constexpr (!WAVE) {
+        I.range(gd.run_off, gd.x_off, g);
+        if constexpr (LPG >= 8) load();
+        if (MODE != GM_PUSH1 || gd.n_temp > 0) I.load(gd, ln % LPG, gd.n_temp > 0 || gd.any_fsrc);
+    }
     {
+        // the layers' parameters into LDS: those this workgroup's grains lie in, or, where a
+        // launch is a few workgroups and only its latency counts, all in one sweep
         typedef unsigned long long u64;
-        const int nw = gd.nl * (int)(sizeof(LayerParams) / sizeof(u64));
+        constexpr int nw = (int)(sizeof(LayerParams) / sizeof(u64));
         const u64* src = reinterpret_cast<const u64*>(gd.lp);
         u64* dst = reinterpret_cast<u64*>(slp);
-        for (int i = threadIdx.x; i < nw; i += blockDim.x) dst[i] = src[i];
+        if constexpr (WAVE) {
+            const int b0 = bl * (256 / LPG), b1 = b0 + 256 / LPG;
+            for (int q = 0; q < gd.nl; q++)
+                if (gd.loff[q] < b1 && gd.loff[q + 1] > b0)
+                    for (int i = threadIdx.x; i < nw; i += blockDim.x) dst[q * nw + i] = src[q * nw + i];
+        } else {
+            for (int i = threadIdx.x; i < gd.nl * nw; i += blockDim.x) dst[i] = src[i];
+        }
     }
     if (a.diag)
         for (int i = threadIdx.x; i < DIAG_STRIDE; i += blockDim.x) red[i] = 0.0;
@@ -747,12 +984,26 @@ __global__ void __launch_bounds__(256) k_grain(GrainData<T> gd, T* __restrict__ 
     const LayerParams& L = slp[k];
     T h[3] = {0, 0, 0};
     double tev[2] = {0, 0};   // grain temperature now and at the next evaluation (moving sources)
+    GrainSums S;
+    if (ngw > 0 && (MODE != GM_PUSH1 || gd.n_temp > 0)) {
+        if constexpr (WAVE)
+            grain_sums<T, LPG>(gd, slp, gw0, ngw, mf, Hr, MODE == GM_PUSH1,
+                               gval + wv * GrainShape<LPG>::doubles(gd.n_temp), S);
+        else
+            grain_sums_lanes<T, LPG>(gd, slp, k, ln % LPG, mf, Hr, MODE == GM_PUSH1, I, S);
+    }
+    if (act) {
+    if constexpr (LPG < 8) load();
     if (MODE != GM_PUSH1) {
-        field_at<T, LPG, TC>(gd, L, k, g, lane, mf, Hr, a.clk ? a.clk[0] + a.t : a.t, mfield, h, tev, P);
+        field_at<T>(gd, L, g, S, Hr != nullptr, a.clk ? a.clk[0] + a.t : a.t, mfield, h, tev, P);
     } else {
 #pragma unroll
         for (int c = 0; c < 3; c++) h[c] = hout[(size_t)c * G + g];
-        if (L.src[1].kind != MRMG_SRC_NONE) src_temp<T, LPG>(gd, L, g, lane, tev);
+        if (L.src[1].kind != MRMG_SRC_NONE) {
+            const double dc = (double)P.cells;
+            tev[0] = S.t[0] / dc + g_temp;
+            if (gd.n_temp > 1) tev[1] = S.t[1] / dc + g_temp;
+        }
     }
     T mo[3] = {0, 0, 0};
     T fsc = 0;   // Ms * ms_scale of the new state: the cell magnetisation factor
@@ -920,6 +1171,7 @@ __global__ void __launch_bounds__(256) k_grain(GrainData<T> gd, T* __restrict__ 
     }
     // the new magnetisation of the grain's cells, for the next field evaluation
     if (MODE != GM_FIELD1 && Mg && w0) store_mg<T, TC>(Mg, G, g, fsc, mo);
+    }
     if (a.diag) {
         __syncthreads();
         for (int i = threadIdx.x; i < DIAG_STRIDE; i += blockDim.x) diag_part[(size_t)bl * DIAG_STRIDE + i] = red[i];
@@ -1116,13 +1368,16 @@ int Engine<T>::scatter(S* m, const double* t0 )
 }
 
 template <typename T>
-template <int MODE, int LPG> void Engine<T>::launch_grain(const StepArgs& a, S* mout)
+template <int MODE, int LPG> int Engine<T>::launch_grain(const StepArgs& a, S* mout)
 {
     const size_t threads = (size_t)G * LPG;
     const unsigned nb8 = (unsigned)(((threads + 255) / 256 + 7) / 8 * 8);
-    hipLaunchKernelGGL((k_grain<S, MODE, LPG, T>), dim3(nb8), dim3(256), 0, c->stream,
+    hipLaunchKernelGGL((k_grain<S, MODE, LPG, T>), dim3(nb8), dim3(256),
+                       LPG <= 2 ? 4 * sizeof(double) * GrainShape<LPG>::doubles(n_temp) : 0, c->stream,
                        gdata(), ma.p, mb.p, dm.p, hthm.p, h.p, demag_on() ? Hr.p : nullptr,
                        demag_on() ? Mg.p : nullptr, a, diag_part.p, mout);
+    HIPCHK(hipGetLastError());
+    return MRMG_OK;
 }
 
 // mout: destination of the corrector (null: ma); t_next: time of the next field
@@ -1133,12 +1388,11 @@ template <int MODE> int Engine<T>::grain(const StepArgs& a, S* mout, double t_ne
     RCHK(src_axes(a.t, t_next));
     RCHK(ev_begin((MODE == GM_HEUN1 || MODE == GM_ROT1 || MODE == GM_FIELD1 || MODE == GM_PUSH1) ? K_GRAIN1
                                                                                              : K_GRAIN2));
-    if (lpg == 4) launch_grain<MODE, 4>(a, mout);
-    else if (lpg == 2) launch_grain<MODE, 2>(a, mout);
-    else if (lpg == 1) launch_grain<MODE, 1>(a, mout);
-    else if (lpg == 16) launch_grain<MODE, 16>(a, mout);
-    else launch_grain<MODE, 8>(a, mout);
-    HIPCHK(hipGetLastError());
+    if (lpg == 4) RCHK((launch_grain<MODE, 4>(a, mout)));
+    else if (lpg == 2) RCHK((launch_grain<MODE, 2>(a, mout)));
+    else if (lpg == 1) RCHK((launch_grain<MODE, 1>(a, mout)));
+    else if (lpg == 16) RCHK((launch_grain<MODE, 16>(a, mout)));
+    else RCHK((launch_grain<MODE, 8>(a, mout)));
     RCHK(ev_end());
     return MRMG_OK;
 }

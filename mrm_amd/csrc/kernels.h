@@ -136,14 +136,18 @@ __host__ __device__ inline size_t tensor_block(int kx, int ko, int ks, int nl, i
 // data.f90:344-353) and write the cell field's sums over them, which the grain kernels add
 // up (get_magnetostatic, field.f90:463-468); no cell array goes to memory.  Runs are
 // numbered grain by grain (each grain's runs contiguous, in the order of its cells) and
-// listed a second time row by row for the row kernels.
+// listed a second time row by row for the row kernels, which write their sums in that order
+// (consecutive lanes, consecutive runs); the grain kernels read them through run_q.
 struct RowRuns {
     const int* row_off;   // [nl*ny + 1]: the runs of row (k, y) are [row_off[k*ny + y], row_off[k*ny + y + 1])
     const int* geo;       // row by row: first x | length << 16
     const int* grain;     // row by row: global grain
-    const int* gm;        // row by row: the run's number in the grain-by-grain order
     int nruns;
 };
+// the row and the layer of a run in one word (GrainData::run_row): no row FFT of 2^24 rows
+// fits a workgroup
+#define RUN_LAYER_SHIFT 24
+#define RUN_ROW_MASK 0xffffff
 
 // The per-context operands of the demag kernels.  A kernel launched for one context takes
 // them by value; a launch over a batch of contexts whose FFT grids and launch shapes are
@@ -154,7 +158,7 @@ template <typename T> struct DemagOps {
     C2<T>* S2;              // spectra of H
     const C2<T>* Tspec;     // tensor spectra
     T* Hcell;               // cell field (mrmg_demag_field only)
-    double* Hr;             // [3][nruns] run sums of the cell field
+    double* Hr;             // [3][nruns] run sums of the cell field, row by row
     RowRuns R;
     int G, pad_;
 };
@@ -183,11 +187,14 @@ template <typename T> struct GrainData {
     const int* gc_off;    // grain -> cells CSR (grain2gridindex): the cell count of grain g
                           // is gc_off[g+1] - gc_off[g]
     const int* run_off;   // grain -> runs CSR (RowRuns' grain-by-grain numbering)
+    // (arrays of their own: as one 16-byte record a run, and one an exchange entry, the
+    // wider loads cost more than they saved, 179 against 161 us in the 2048x2048x8 write)
     const int* run_geo;   //   first x | length << 16
-    const int* run_row;   //   row y within the grain's layer
+    const int* run_row;   //   row y within the grain's layer | layer << RUN_LAYER_SHIFT
+    const int* run_q;     //   the run's number in the row-by-row order (the run sums' order)
     int nruns;
     // exchange CSR, per grain the intralayer entries, then those to the layer above, then
-    // to the layer below; x_nb/x_w carry one spare entry at the end
+    // to the layer below, and one spare entry at the end
     const int* x_off; const int* x_nb; const T* x_w;
     const LayerParams* lp;
     int nl;
@@ -196,7 +203,10 @@ template <typename T> struct GrainData {
     const double* lam;
     const double* temp;
     const double* tabs;   // READ_SCALE table nodes and values of every layer
-    int any_src;          // some layer has a moving source
+    int any_fsrc;         // some layer has a field table
+    int n_temp;           // temperature sources: 0 none, 1 needed at the evaluation, 2 also at the next one
+    int all_sg;           // every temperature source is a super-Gaussian
+    int loff[MRMG_MAX_LAYERS + 1];     // first grain of each layer, and G
     SrcAxes ax;
 };
 
