@@ -189,7 +189,7 @@ struct EngineBase {
     virtual int kernel_stats(mrmg_kstat* out, int max, int* n) = 0;
     virtual int readback(const mrmg_sensor* s, int n_pos, const double* xpos, const double* ypos, double* out) = 0;
     virtual int readback_into(const mrmg_sensor* s, int n_pos, const double* xpos, const double* ypos, double* out,
-                              double* plane, double* pos, double* dout) = 0;
+                              double* plane, double* pos, double* dout, long long* odd) = 0;
     virtual int switch_arm(int enable, const double* dir, double thr) = 0;
     virtual int switch_read(int k, int64_t* step, double* t, double* hap) = 0;
     virtual int time_class(int cls, int reps, double* ms) = 0;
@@ -334,7 +334,7 @@ struct Engine : EngineBase {
     size_t lds_rowT = 0, lds_colT = 0;
     DBuf<double> noise_buf, diag_part, stats;
     // switching record and readback buffers (allocated on first use)
-    DBuf<long long> sw_step;
+    DBuf<long long> sw_step, rb_odd;
     DBuf<double> sw_t, sw_h, rb_plane, rb_pos, rb_out;
     bool sw_on = false;
     double sw_dir[3] = {0, 0, 0}, sw_thr = 0;
@@ -412,7 +412,7 @@ struct Engine : EngineBase {
         b += noise_buf.bytes() + diag_part.bytes() + stats.bytes();
         b += src_pos.bytes() + src_vals.bytes() + ax_xa.bytes() + ax_xc.bytes() + ax_ya.bytes() + ax_yb.bytes() +
              ax_xi.bytes() + ax_yi.bytes() + tlast.bytes();
-        b += sw_step.bytes() + sw_t.bytes() + sw_h.bytes() + rb_plane.bytes() + rb_pos.bytes() + rb_out.bytes();
+        b += sw_step.bytes() + sw_t.bytes() + sw_h.bytes() + rb_plane.bytes() + rb_pos.bytes() + rb_out.bytes() + rb_odd.bytes();
         b += btab_buf.bytes() + clk_buf.bytes();
         return b;
     }
@@ -1449,9 +1449,10 @@ struct Engine : EngineBase {
         if (rb_plane.n < nxy) RCHK(rb_plane.alloc(nxy));
         if (rb_pos.n < 2 * (size_t)n_pos) RCHK(rb_pos.alloc(2 * (size_t)n_pos));
         if (rb_out.n < (size_t)n_pos) RCHK(rb_out.alloc(n_pos));
-        return readback_into(sn, n_pos, xpos, ypos, out, rb_plane.p, rb_pos.p, rb_out.p);
+        if (rb_odd.n < 1) RCHK(rb_odd.alloc(1));
+        return readback_into(sn, n_pos, xpos, ypos, out, rb_plane.p, rb_pos.p, rb_out.p, rb_odd.p);
     }
-    int readback_into(const mrmg_sensor* sn, int n_pos, const double* xpos, const double* ypos, double* out, double* plane, double* pos, double* dout) override;
+    int readback_into(const mrmg_sensor* sn, int n_pos, const double* xpos, const double* ypos, double* out, double* plane, double* pos, double* dout, long long* odd) override;
     int switch_arm(int enable, const double* dir, double thr) override;
     int switch_mark(long long step, double t);
     int switch_read(int k, int64_t* step, double* t, double* hap) override

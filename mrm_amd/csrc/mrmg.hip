@@ -25,9 +25,9 @@ int set_err(int code, const char* fmt, ...)
 }
 
 // Scratch of the allocation-free readback: the plane, then the head positions (x, y), then
-// the outputs.  Host code never passes this name to a kernel (it is a host-side stand-in);
+// the outputs, and one word for the plane's non-finite mark.  Host code never passes this name to a kernel (it is a host-side stand-in);
 // it uses the device address hipGetSymbolAddress returns for the current device.
-#define RB_SCRATCH_DOUBLES ((size_t)MRMG_NOALLOC_PLANE_MAX + 3 * (size_t)MRMG_NOALLOC_POS_MAX)
+#define RB_SCRATCH_DOUBLES ((size_t)MRMG_NOALLOC_PLANE_MAX + 3 * (size_t)MRMG_NOALLOC_POS_MAX + 1)
 static __device__ __align__(256) double scratch[RB_SCRATCH_DOUBLES];
 
 // ------------------------------------------------------------------------- C ABI
@@ -638,7 +638,8 @@ int mrmg_readback_noalloc(mrmg_ctx* c, const mrmg_sensor* s, int n_pos, const do
     double* plane = sp;
     double* pos = sp + MRMG_NOALLOC_PLANE_MAX;
     double* dout = pos + 2 * (size_t)MRMG_NOALLOC_POS_MAX;
-    return c->eng->readback_into(s, n_pos, xpos, ypos, out, plane, pos, dout);
+    return c->eng->readback_into(s, n_pos, xpos, ypos, out, plane, pos, dout,
+                                 reinterpret_cast<long long*>(dout + MRMG_NOALLOC_POS_MAX));
 }
 
 int mrmg_switch_arm(mrmg_ctx* c, int enable, const double* dir, double thr)
