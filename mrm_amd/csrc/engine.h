@@ -413,7 +413,7 @@ struct Engine : EngineBase {
         b += src_pos.bytes() + src_vals.bytes() + ax_xa.bytes() + ax_xc.bytes() + ax_ya.bytes() + ax_yb.bytes() +
              ax_xi.bytes() + ax_yi.bytes() + tlast.bytes();
         b += sw_step.bytes() + sw_t.bytes() + sw_h.bytes() + rb_plane.bytes() + rb_pos.bytes() + rb_out.bytes() + rb_odd.bytes();
-        b += btab_buf.bytes() + clk_buf.bytes();
+        b += btab_buf.bytes() + clk_buf.bytes() + gtab_buf.bytes();
         return b;
     }
     bool has_tensor() const override { return tensor_ok; }
@@ -1140,6 +1140,9 @@ struct Engine : EngineBase {
 
     template <int MODE, int LPG> int launch_grain(const StepArgs& a, S* mout);
     template <int MODE> int grain(const StepArgs& a, S* mout = nullptr, double t_next = 0.0);
+    GrainOps<S, T> grain_ops(unsigned long long seed, const double* clk) const;
+    template <int MODE> int grain_batch(const GrainOps<S, T>* tab, int n, int most, const StepArgs& a);
+    DBuf<GrainOps<S, T>> gtab_buf;   // a batch's table, held by its lead context
 
     // per-layer reductions of the last diag-enabled grain launch
     struct LayerRed {
@@ -1523,11 +1526,11 @@ struct Engine : EngineBase {
 
 // ---------------------------------------------------------------------------------------
 // Serving: fixed-dt steps of a batch of contexts with equal grids and launch shapes.  The
-// members' work runs on the first member's stream: per stage each member's grain kernel,
-// and each demag kernel class once for all members (their operands in a device table,
-// blockIdx.z the member).  The time and thermal step counter of every member live in a
-// device clock, so one step is the same launch sequence every time; with graph set it is
-// captured once as a hipGraph and replayed n_steps times.  Each member gets the values
+// members' work runs on the first member's stream: per stage each demag kernel class, and
+// the grain kernel, once for all members (their operands in device tables).  The time and
+// thermal step counter of every member live in a device clock, so one step is the same
+// launch sequence every time; with graph set it is captured once as a hipGraph and replayed
+// n_steps times.  Each member gets the values
 // its own mrmg_step with Philox noise (or none) would give: the same kernels, the same
 // thermal normals (drawn in the grain kernel from the member's seed and step) and the
 // host loop's time arithmetic, done on the device.
@@ -1619,6 +1622,27 @@ int batch_step(std::vector<Engine<T>*>& M, const mrmg_step_params* P, int graph,
         a[b].seed = P[b].seed;
         a[b].clk = L.clk_buf.p + 2 * b;
     }
+    // a stage's grain kernels: one launch for all members where they split their grains alike
+    // (and keep their buffers from step to step), else one each
+    int most = 0;
+    bool together = type < 0 && B > 1 && (L.lpg == 1 || L.lpg == 4 || L.lpg == 8);
+    for (int b = 0; b < B; b++) {
+        most = std::max(most, M[b]->G);
+        together = together && M[b]->lpg == L.lpg;
+    }
+    std::vector<GrainOps<double, T>> gtab;
+    if (together) {
+        for (int b = 0; b < B; b++) gtab.push_back(M[b]->grain_ops(P[b].seed, L.clk_buf.p + 2 * b));
+        if (L.gtab_buf.n < (size_t)B) RCHK(L.gtab_buf.alloc(B));
+        HIPCHK(hipMemcpyAsync(L.gtab_buf.p, gtab.data(), sizeof(gtab[0]) * B, hipMemcpyHostToDevice, s));
+    }
+    auto grain_all = [&](auto mode, double t, double dts) -> int {
+        constexpr int MODE = decltype(mode)::value;
+        for (int b = 0; b < B; b++) { a[b].t = t; a[b].dts = dts; }
+        if (together) return L.template grain_batch<MODE>(L.gtab_buf.p, B, most, a[0]);
+        for (int b = 0; b < B; b++) RCHK(M[b]->template grain<MODE>(a[b], nullptr, 0.0));
+        return MRMG_OK;
+    };
     auto demag_all = [&]() -> int {
         if (!L.demag_on()) return MRMG_OK;
         L.btab = L.btab_buf.p;
@@ -1632,26 +1656,14 @@ int batch_step(std::vector<Engine<T>*>& M, const mrmg_step_params* P, int graph,
     auto one_step = [&]() -> int {
         if (type == -3) {
             RCHK(demag_all());
-            for (int b = 0; b < B; b++) {
-                a[b].t = 0.0; a[b].dts = dt;
-                RCHK(M[b]->template grain<GM_HEUN1>(a[b], nullptr, 0.0));
-            }
+            RCHK(grain_all(std::integral_constant<int, GM_HEUN1>(), 0.0, dt));
             RCHK(demag_all());
-            for (int b = 0; b < B; b++) {
-                a[b].t = dt;
-                RCHK(M[b]->template grain<GM_HEUN2>(a[b], nullptr, 0.0));
-            }
+            RCHK(grain_all(std::integral_constant<int, GM_HEUN2>(), dt, dt));
         } else if (type < 0) {
             RCHK(demag_all());
-            for (int b = 0; b < B; b++) {
-                a[b].t = 0.0; a[b].dts = dt * 0.5;
-                RCHK(M[b]->template grain<GM_ROT1>(a[b], nullptr, 0.0));
-            }
+            RCHK(grain_all(std::integral_constant<int, GM_ROT1>(), 0.0, dt * 0.5));
             RCHK(demag_all());
-            for (int b = 0; b < B; b++) {
-                a[b].t = dt * 0.5; a[b].dts = dt;
-                RCHK(M[b]->template grain<GM_ROT2>(a[b], nullptr, 0.0));
-            }
+            RCHK(grain_all(std::integral_constant<int, GM_ROT2>(), dt * 0.5, dt));
         } else {
             RCHK(demag_all());
             for (int b = 0; b < B; b++) {

@@ -909,10 +909,10 @@ __device__ __forceinline__ void rot_push(int type, T scale1, T scale2, const T* 
 
 
 template <typename T, int MODE, int LPG, typename TC>
-__global__ void __launch_bounds__(256) k_grain(GrainData<T> gd, T* __restrict__ ma, T* __restrict__ mb,
-                                               T* __restrict__ dm, T* __restrict__ hthm, T* __restrict__ hout,
-                                               const double* __restrict__ Hr, TC* __restrict__ Mg,
-                                               StepArgs a, double* __restrict__ diag_part, T* __restrict__ mc)
+__device__ __forceinline__ void grain_body(const GrainData<T>& gd, T* __restrict__ ma, T* __restrict__ mb,
+                                           T* __restrict__ dm, T* __restrict__ hthm, T* __restrict__ hout,
+                                           const double* __restrict__ Hr, TC* __restrict__ Mg, const StepArgs& a,
+                                           double* __restrict__ diag_part, T* __restrict__ mc)
 {
     // grid padded to a multiple of 8: each XCD takes a contiguous range of grains, so the
     // cell lines neighbouring grains share stay in one L2
@@ -1176,6 +1176,28 @@ __global__ void __launch_bounds__(256) k_grain(GrainData<T> gd, T* __restrict__ 
         __syncthreads();
         for (int i = threadIdx.x; i < DIAG_STRIDE; i += blockDim.x) diag_part[(size_t)bl * DIAG_STRIDE + i] = red[i];
     }
+}
+
+template <typename T, int MODE, int LPG, typename TC>
+__global__ void __launch_bounds__(256) k_grain(GrainData<T> gd, T* __restrict__ ma, T* __restrict__ mb,
+                                               T* __restrict__ dm, T* __restrict__ hthm, T* __restrict__ hout,
+                                               const double* __restrict__ Hr, TC* __restrict__ Mg,
+                                               StepArgs a, double* __restrict__ diag_part, T* __restrict__ mc)
+{
+    grain_body<T, MODE, LPG, TC>(gd, ma, mb, dm, hthm, hout, Hr, Mg, a, diag_part, mc);
+}
+
+// One stage of every member of a batch (blockIdx.y the member): a member of some thousand
+// grains fills a small part of the chip, and sixteen launches of it one after the other cost
+// sixteen latencies (16 contexts of 256x256x2, 7 846 grains each: 64 / 53 us a stage against
+// 117 / 101).  a: the stage's times and the push, equal for all; seed and clock are the member's.
+template <typename T, int MODE, int LPG, typename TC>
+__global__ void __launch_bounds__(256) k_grain_batch(const GrainOps<T, TC>* __restrict__ tab, StepArgs a)
+{
+    const GrainOps<T, TC>& o = tab[blockIdx.y];
+    a.seed = o.seed;
+    a.clk = o.clk;
+    grain_body<T, MODE, LPG, TC>(o.gd, o.ma, o.mb, o.dm, o.hthm, o.h, o.Hr, o.Mg, a, nullptr, nullptr);
 }
 
 // llg()'s loop-top statistics (llg.f90:217-237) of layer blockIdx.x: the volume-weighted
@@ -1448,6 +1470,41 @@ template <int MODE> int Engine<T>::grain(const StepArgs& a, S* mout, double t_ne
     return MRMG_OK;
 }
 
+// this context's operands in a batch's grain launches
+template <typename T>
+GrainOps<double, T> Engine<T>::grain_ops(unsigned long long seed, const double* clk) const
+{
+    GrainOps<S, T> o{};
+    o.gd = gdata();
+    o.ma = ma.p; o.mb = mb.p; o.dm = dm.p; o.hthm = hthm.p; o.h = h.p;
+    o.Hr = demag_on() ? Hr.p : nullptr;
+    o.Mg = demag_on() ? Mg.p : nullptr;
+    o.seed = seed;
+    o.clk = clk;
+    return o;
+}
+
+// one stage of the n members of the device table tab, whose lanes per grain are this
+// context's; most: the largest number of grains.  MRMG_ERR_UNSUPPORTED (without a message)
+// for a number of lanes that only single launches are built for.
+template <typename T>
+template <int MODE> int Engine<T>::grain_batch(const GrainOps<S, T>* tab, int n, int most, const StepArgs& a)
+{
+    const unsigned nb8 = (unsigned)((((size_t)most * lpg + 255) / 256 + 7) / 8 * 8);
+    const dim3 g(nb8, (unsigned)n);
+    if (lpg == 1)
+        hipLaunchKernelGGL((k_grain_batch<S, MODE, 1, T>), g, dim3(256),
+                           4 * sizeof(double) * GrainShape<1>::doubles(n_temp), c->stream, tab, a);
+    else if (lpg == 4)
+        hipLaunchKernelGGL((k_grain_batch<S, MODE, 4, T>), g, dim3(256), 0, c->stream, tab, a);
+    else if (lpg == 8)
+        hipLaunchKernelGGL((k_grain_batch<S, MODE, 8, T>), g, dim3(256), 0, c->stream, tab, a);
+    else
+        return MRMG_ERR_UNSUPPORTED;
+    HIPCHK(hipGetLastError());
+    return MRMG_OK;
+}
+
 // llg()'s loop-top statistics of the current state and h, into stats
 template <typename T>
 int Engine<T>::layer_stats()
@@ -1552,13 +1609,18 @@ int launch_copy16(hipStream_t s, unsigned grid, const uint4* a, uint4* b, size_t
     template int Engine<T>::scatter(double*, const double*);                                               \
     template int Engine<T>::layer_stats();                                                                 \
     template int Engine<T>::readback_into(const mrmg_sensor*, int, const double*, const double*, double*,   \
-                                          double*, double*, double*);                                       \
+                                          double*, double*, double*, long long*);                           \
     template int Engine<T>::switch_arm(int, const double*, double);                                        \
     template int Engine<T>::switch_mark(long long, double);                                                \
     template int Engine<T>::grain<GM_HEUN1>(const StepArgs&, double*, double);                             \
     template int Engine<T>::grain<GM_HEUN2>(const StepArgs&, double*, double);                             \
     template int Engine<T>::grain<GM_ROT1>(const StepArgs&, double*, double);                              \
     template int Engine<T>::grain<GM_ROT2>(const StepArgs&, double*, double);                              \
+    template GrainOps<double, T> Engine<T>::grain_ops(unsigned long long, const double*) const;            \
+    template int Engine<T>::grain_batch<GM_HEUN1>(const GrainOps<double, T>*, int, int, const StepArgs&);  \
+    template int Engine<T>::grain_batch<GM_HEUN2>(const GrainOps<double, T>*, int, int, const StepArgs&);  \
+    template int Engine<T>::grain_batch<GM_ROT1>(const GrainOps<double, T>*, int, int, const StepArgs&);   \
+    template int Engine<T>::grain_batch<GM_ROT2>(const GrainOps<double, T>*, int, int, const StepArgs&);   \
     template int Engine<T>::grain<GM_FIELD1>(const StepArgs&, double*, double);                            \
     template int Engine<T>::grain<GM_PUSH1>(const StepArgs&, double*, double);
 MRMG_INST(float)

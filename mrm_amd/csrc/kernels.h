@@ -245,3 +245,14 @@ struct StepArgs {
     // the evaluation time is clk[0] + t and the thermal counter clk[1] + step
     const double* clk;
 };
+
+// The operands of one member of a batched grain launch (a device table of them, indexed by
+// blockIdx.y).
+template <typename T, typename TC> struct GrainOps {
+    GrainData<T> gd;
+    T *ma, *mb, *dm, *hthm, *h;
+    const double* Hr;
+    TC* Mg;
+    unsigned long long seed;
+    const double* clk;
+};
