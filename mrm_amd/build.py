@@ -12,6 +12,7 @@ CSRC = os.path.join(HERE, "csrc")
 # (source, object, extra flags): the demag units once per precision form
 UNITS = [("mrmg.hip", "mrmg.o", []), ("grain.hip", "grain.o", []), ("tensor.hip", "tensor.o", []),
          ("demag.hip", "demag_f32.o", ["-DMRMG_FORM=float"]), ("demag.hip", "demag_f64.o", ["-DMRMG_FORM=double"]),
+         ("colprod.hip", "colprod_f64.o", []), ("rowsplit.hip", "rowsplit_f64.o", []),
          ("column.hip", "column_f32a.o", ["-DMRMG_FORM=float", "-DMRMG_COL_PART=1"]),
          ("column.hip", "column_f32b.o", ["-DMRMG_FORM=float", "-DMRMG_COL_PART=2"]),
          ("column.hip", "column_f64a.o", ["-DMRMG_FORM=double", "-DMRMG_COL_PART=1"]),

@@ -610,8 +610,9 @@ static void launch_prod_offsets(bool sym, bool bat, bool nt, dim3 g, hipStream_t
 template <typename T>
 int Engine<T>::launch_class(int cls)
 {
-    // row kernels: the media rows; column and product kernels: the FFT grid
-    const int ny = c->ny, fy = c->fy, nl = c->nl, nxh = c->nxh;
+    // row kernels: the media rows; column and product kernels: the columns as they are laid
+    // out (RowSplit), nxh of fy values unless the transform is split
+    const int ny = c->ny, fy = vL(), nl = c->nl, nxh = vnx();
     const unsigned z = btab ? (unsigned)bn : 1u;
     const dim3 grow((ny + 1) / 2, nl, z), growT(rowT_blocks(), 1, z), blk(row_threads), b256(256);
     const int ncols = 3 * nl * nxh;
@@ -620,10 +621,14 @@ int Engine<T>::launch_class(int cls)
         return set_err(MRMG_ERR_STATE, "batched demag launches run without wave-local FFTs or cell output");
     switch (cls) {
     case K_ROW_FWD:
+        if constexpr (sizeof(T) == 8)
+            if (subR > 1) return launch_rowS(false, growT, blk);
         if (tl || split) LAUNCH_E(maxb_rowT, launch_rowT_fwd, growT, blk);
         else LAUNCH_E(maxb_row, launch_row_fwd, grow, blk);
         break;
     case K_COL: {
+        if constexpr (sizeof(T) == 8)
+            if (split && colp) return launch_colp();
         if (split) return set_err(MRMG_ERR_STATE, "the split path has no fused column kernel");
         const int nb8 = (nxh * kg + 7) / 8 * 8;
         if (nslot == 6) LAUNCH_E(maxb_col, launch_col_sym, nb8);
@@ -667,6 +672,8 @@ int Engine<T>::launch_class(int cls)
         break;
     }
     case K_ROW_INV:
+        if constexpr (sizeof(T) == 8)
+            if (subR > 1) return launch_rowS(true, growT, blk);
         if (tl || split) LAUNCH_E(maxb_rowT, launch_rowT_inv, growT, blk);
         else LAUNCH_E(maxb_row, launch_row_inv, grow, blk);
         break;
@@ -697,11 +704,11 @@ template <int MB> void Engine<T>::launch_colT_fwd(dim3 g, dim3 b)
 {
     const DemagOps<T> o = ops();
     if (btab)
-        hipLaunchKernelGGL((k_colT<T, MB, false, true>), g, b, lds_colT, c->stream, o, btab, c->fy, c->ny,
-                           3 * c->nl * c->nxh, CBc, pcol, twy.p);
+        hipLaunchKernelGGL((k_colT<T, MB, false, true>), g, b, lds_colT, c->stream, o, btab, vL(), col_rows(),
+                           3 * c->nl * vnx(), CBc, pcol, twy.p);
     else
-        hipLaunchKernelGGL((k_colT<T, MB, false>), g, b, lds_colT, c->stream, o, btab, c->fy, c->ny,
-                           3 * c->nl * c->nxh, CBc, pcol, twy.p);
+        hipLaunchKernelGGL((k_colT<T, MB, false>), g, b, lds_colT, c->stream, o, btab, vL(), col_rows(),
+                           3 * c->nl * vnx(), CBc, pcol, twy.p);
 }
 
 template <typename T>
@@ -709,11 +716,11 @@ template <int MB> void Engine<T>::launch_colT_inv(dim3 g, dim3 b)
 {
     const DemagOps<T> o = ops();
     if (btab)
-        hipLaunchKernelGGL((k_colT<T, MB, true, true>), g, b, lds_colT, c->stream, o, btab, c->fy, c->ny,
-                           3 * c->nl * c->nxh, CBc, pcol, twy.p);
+        hipLaunchKernelGGL((k_colT<T, MB, true, true>), g, b, lds_colT, c->stream, o, btab, vL(), col_rows(),
+                           3 * c->nl * vnx(), CBc, pcol, twy.p);
     else
-        hipLaunchKernelGGL((k_colT<T, MB, true>), g, b, lds_colT, c->stream, o, btab, c->fy, c->ny,
-                           3 * c->nl * c->nxh, CBc, pcol, twy.p);
+        hipLaunchKernelGGL((k_colT<T, MB, true>), g, b, lds_colT, c->stream, o, btab, vL(), col_rows(),
+                           3 * c->nl * vnx(), CBc, pcol, twy.p);
 }
 
 template <typename T>

@@ -328,6 +328,12 @@ struct Engine : EngineBase {
     bool pre = false;
     bool wv = false;   // wave-local FFTs in the transposing row kernels and the path-2 column kernel
     int TYr = 8, CBc = 1, maxb_rowT = 4, maxb_colT = 4;
+    // the split of the column transform (RowSplit): its radix, the media rows of a group; the
+    // one-kernel column path (colprod.hip) and its launch shape
+    int subR = 1, subRm = 1, colp_threads = 256;
+    bool colp = false;
+    size_t lds_colp = 0;
+    DBuf<C2<T>> tws;
     // FFT plans of the step's row and column transforms and their largest radix
     FFTPlan prow{}, pcol{};
     int row_radix = 16, col_radix = 16;
@@ -407,7 +413,7 @@ struct Engine : EngineBase {
              hk2.bytes() + uni.bytes() + cub.bytes() + happ.bytes() + sigma.bytes() + sigma_llb.bytes() + vol.bytes() +
              lp.bytes() + tc.bytes() + lam.bytes() + temp.bytes();
         b += ma.bytes() + mb.bytes() + mc.bytes() + dm.bytes() + hthm.bytes() + h.bytes();
-        b += S1.bytes() + S2.bytes() + Tspec.bytes() + twx.bytes() + twy.bytes() + Hcell.bytes() +
+        b += S1.bytes() + S2.bytes() + Tspec.bytes() + twx.bytes() + twy.bytes() + tws.bytes() + Hcell.bytes() +
              slot2c.bytes();
         b += noise_buf.bytes() + diag_part.bytes() + stats.bytes();
         b += src_pos.bytes() + src_vals.bytes() + ax_xa.bytes() + ax_xc.bytes() + ax_ya.bytes() + ax_yb.bytes() +
@@ -464,8 +470,11 @@ struct Engine : EngineBase {
             return set_err(MRMG_ERR_UNSUPPORTED, "grid %dx%dx%d: a row or column FFT does not fit one workgroup", nx, ny,
                            nl);
         split = !fused_ok;
+        if (split) RCHK(choose_split());
         // long rows run fastest with the widest row workgroups (measured at 2048 points)
-        if (nx >= 1024) row_threads = 256;
+        // and so do the split transform's row kernels (512x4096x4 FP64: 122 / 126 us with 256
+        // threads against 135 / 151 with 128)
+        if (nx >= 1024 || (subR > 1 && TYr_eff() * nx >= 4096)) row_threads = 256;
         RCHK(shapes());
         RCHK(lds_attr());
         RCHK(S1.alloc((size_t)nl * 3 * ny * nxh));
@@ -476,6 +485,77 @@ struct Engine : EngineBase {
         if (c->open) HIPCHK(hipMemsetAsync(S1.p, 0, S1.bytes(), c->stream));
         kg = 1;
         return MRMG_OK;
+    }
+
+    // The split of the column transform over the row kernels (RowSplit), for which the columns
+    // left between them go through one kernel (forward transform, product and inverse in LDS,
+    // colprod.hip) instead of three passes over memory.  FP64 only: in FP32 the other order of
+    // the transform's steps moves a run's mean magnetisation by more than 1e-9.  Taken with the
+    // largest radix for which
+    // * a column keeps 256 values, one a thread of the product (FP32, columns of 1024 values
+    //   of 8 layers: radix 4 takes 138 us a field for the columns, radix 8 190);
+    // * 3 n_lay columns are at most 112 KB (512x4096x4: radix 8 of 98 KB, one workgroup a CU,
+    //   271 us a field against 380 in three kernels; rows 122 / 126 against 102 / 105);
+    // * the product's registers hold the layers (4);
+    // * the row kernels' rows take at most 4096 transform elements (70 KB; 64 a thread with
+    //   the fewest threads that can be asked for).
+    int choose_split()
+    {
+        const int nl = c->nl, fy = c->fy;
+        subR = subRm = 1;
+        colp = false;
+        if (sizeof(T) != 8 || nl > 4) return MRMG_OK;
+        for (int R = 8; R >= (c->open ? 2 : 1) && !colp; R /= 2) {
+            const int L = fy / R, rm = c->open ? R / 2 : R, ty = std::max(TYr, rm);
+            FFTPlan q;
+            if (fy % R != 0 || L < 256 || !factorize(L, q)) continue;
+            const size_t lc = sizeof(T) * 2 * LPN(3 * nl * L);
+            const int th = lc > 56 * 1024 ? 512 : 256, e = pick_e(3 * nl, q, th);
+            if (lc > 112 * 1024 || ty / 2 * c->fx > 4096 || ty > 16) continue;
+            if (pick_e(ty / 2, c->px, 256) < 0 || e < 0 || e > 32) continue;
+            subR = R;
+            subRm = rm;
+            colp = true;
+            colp_threads = th;
+            lds_colp = lc;
+            pcol = q;
+        }
+        if (!colp) return MRMG_OK;
+        RCHK(upload_twiddles(pcol, twy));
+        lds_rowT = sizeof(T) * 2 * LPN((TYr_eff() / 2) * c->fx);
+        CBc = std::max(1, std::min(16, 2048 / pcol.n));
+        CBc = std::min(CBc, 3 * nl * vnx());
+        lds_colT = sizeof(T) * 2 * LPN(CBc * pcol.n);
+        if (subR > 1) {
+            // w_fy^(r y') at y' R + r
+            const std::vector<C2<double>> w = twiddle_table(fy);
+            std::vector<C2<T>> t(fy);
+            for (int y = 0; y < pcol.n; y++)
+                for (int r = 0; r < subR; r++) {
+                    const C2<double> v = w[(size_t)r * y];
+                    t[(size_t)y * subR + r] = {(T)v.x, (T)v.y};
+                }
+            RCHK(tws.upload(t.data(), t.size(), c->stream));
+            HIPCHK(hipStreamSynchronize(c->stream));
+        }
+        return MRMG_OK;
+    }
+    // the columns as laid out: vnx() per plane, of vL() values
+    int vL() const { return c->fy / subR; }
+    int vnx() const { return c->nxh * subR; }
+    // the rows of a column that the row kernels write and read
+    int col_rows() const { return subR > 1 ? vL() : c->ny; }
+    // rows of a transposing row workgroup: a split one takes whole groups
+    int TYr_eff() const { return std::max(TYr, subRm); }
+    RowSplit<T> row_split() const
+    {
+        RowSplit<T> r;
+        r.R = subR;
+        r.Rm = subRm;
+        r.L = vL();
+        r.Y = TYr_eff() / subRm;
+        r.tw = tws.p;
+        return r;
     }
 
     // the twiddle table of plan q (plan_twiddles), rounded once to T, into d; the stream
@@ -497,8 +577,8 @@ struct Engine : EngineBase {
         const int nl = c->nl, ny = c->fy;
         // wave-local transforms: a lane's bound covers its wave's run of ceil(B / waves)
         auto row_e = [&]() {
-            const int nw = row_threads / 64, b = TYr / 2;
-            return wv ? pick_e((b + nw - 1) / nw, c->px, 64) : pick_e(b, c->px, row_threads);
+            const int nw = row_threads / 64, b = TYr_eff() / 2;
+            return wv && subR == 1 ? pick_e((b + nw - 1) / nw, c->px, 64) : pick_e(b, c->px, row_threads);
         };
         if (split || tl) {
             maxb_rowT = row_e();
@@ -507,7 +587,7 @@ struct Engine : EngineBase {
                                row_threads);
         }
         if (split || pre) {
-            maxb_colT = pick_e(CBc, c->py, 256);
+            maxb_colT = pick_e(CBc, pcol, 256);
             if (maxb_rowT < 0 || maxb_colT < 0)
                 return set_err(MRMG_ERR_UNSUPPORTED, "grid %dx%dx%d: split-path FFT too large for %d threads", c->fx, ny,
                                nl, row_threads);
@@ -574,7 +654,7 @@ struct Engine : EngineBase {
         } else if (k == "row_radix" || k == "col_radix") {
             if (v != 4 && v != 8 && v != 16) return set_err(MRMG_ERR_ARG, "%s must be 4, 8 or 16", k.c_str());
             FFTPlan q;
-            if (!factorize(k == "row_radix" ? c->fx : c->fy, q, v) || q.nfac > MRMG_MAX_FAC)
+            if (!factorize(k == "row_radix" ? c->fx : vL(), q, v) || q.nfac > MRMG_MAX_FAC)
                 return set_err(MRMG_ERR_UNSUPPORTED, "%s %d: no plan", k.c_str(), v);
             if (k == "row_radix") {
                 RCHK(upload_twiddles(q, twx));
@@ -587,8 +667,9 @@ struct Engine : EngineBase {
             }
         } else if (k == "row_block") {
             if (v != 2 && v != 4 && v != 8) return set_err(MRMG_ERR_ARG, "row_block must be 2, 4 or 8");
-            const size_t l = sizeof(T) * 2 * LPN((v / 2) * c->fx);
-            if (l > 160 * 1024 || pick_e(v / 2, c->px, 256) < 0)
+            const int ve = std::max(v, subRm);
+            const size_t l = sizeof(T) * 2 * LPN((ve / 2) * c->fx);
+            if (l > 160 * 1024 || pick_e(ve / 2, c->px, 256) < 0)
                 return set_err(MRMG_ERR_UNSUPPORTED, "row_block %d does not fit LDS", v);
             const int ot = TYr;
             const size_t ol = lds_rowT;
@@ -1075,8 +1156,9 @@ struct Engine : EngineBase {
         static const int fused[3] = {K_ROW_FWD, K_COL, K_ROW_INV};
         static const int splitc[5] = {K_ROW_FWD, K_COLF, K_PROD, K_COLI, K_ROW_INV};
         static const int prec[4] = {K_ROW_FWD, K_COLF, K_COL, K_ROW_INV};
-        const int* seq = split ? splitc : pre ? prec : fused;
-        const int n = split ? 5 : pre ? 4 : 3;
+        const bool one = split && colp && toep && nslot == 6;
+        const int* seq = one ? fused : split ? splitc : pre ? prec : fused;
+        const int n = one ? 3 : split ? 5 : pre ? 4 : 3;
         for (int i = 0; i < n; i++) {
             RCHK(ev_begin(seq[i]));
             RCHK(launch_class(seq[i]));
@@ -1128,7 +1210,13 @@ struct Engine : EngineBase {
     // against 454 us); smaller problems keep them cacheable.
     bool prod_streams() const { return S1.bytes() + S2.bytes() + Tspec.bytes() > (size_t)256 << 20; }
     // transposing row kernels: (ny/TY) * 3 n_lay blocks on a 1D grid padded to a multiple of 8
-    unsigned rowT_blocks() const { return (unsigned)(((c->ny + TYr - 1) / TYr * 3 * c->nl + 7) / 8 * 8); }
+    unsigned rowT_blocks() const
+    {
+        const int per = TYr_eff() / subRm, n = subR > 1 ? vL() : c->ny;   // y' a workgroup, y' in all
+        return (unsigned)(((n + per - 1) / per * 3 * c->nl + 7) / 8 * 8);
+    }
+    int launch_colp();
+    int launch_rowS(bool inv, dim3 g, dim3 b);   // the split transform's row kernels (rowsplit.hip)
     template <int MB> void launch_rowT_fwd(dim3 g, dim3 b);
     template <int MB> void launch_colT_fwd(dim3 g, dim3 b);
     template <int MB> void launch_colT_inv(dim3 g, dim3 b);

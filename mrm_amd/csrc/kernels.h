@@ -163,6 +163,20 @@ template <typename T> struct DemagOps {
     int G, pad_;
 };
 
+// The column transform split over the row kernels (R > 1): a column of N = R L rows takes
+// its first radix-R step (decimation in frequency) where the row r2c holds the R rows y' +
+// q L of it, and the last inverse one in the row c2r, so that between them each (kx, r) is a
+// column of its own of length L:
+//   X_r[y'] = w_N^(r y') sum_q w_R^(r q) x[y' + q L],   Xhat[R s + r] = DFT_L(X_r)[s].
+// The spectra and the tensor are laid out as R nxh columns of L values, column r nxh + kx.
+// Rm: the rows q < Rm of each group that are media rows (R, or R/2 for open boundaries, whose
+// upper half is padding); Y: values of y' per row workgroup (Rm Y rows); tw[y' R + r] =
+// w_N^(r y').
+template <typename T> struct RowSplit {
+    int R, Rm, L, Y;
+    const C2<T>* tw;
+};
+
 // rows of the grain state buffers
 #define ST_MAG 3
 #define ST_MSC 4

@@ -173,18 +173,21 @@ __global__ void __launch_bounds__(256) k_tensor_cols(C2<double>* __restrict__ TC
 
 // Regroup the tensor spectra into Tspec[kx][q][slot][ky] and round to T: q runs over the
 // stored blocks (tensor_block) and real[q] is the real block (9 planes of TC) it comes from.
+// R > 1: the columns of a split transform (RowSplit), column r nxh + kx of ny / R values
+// with ky = R s + r.
 template <typename T>
 __global__ void k_tensor_pack(const C2<double>* __restrict__ TC, C2<T>* __restrict__ Tspec, int ny, int nxh,
-                              int nq, int nslot, const int* __restrict__ slot2c, const int* __restrict__ real)
+                              int nq, int nslot, const int* __restrict__ slot2c, const int* __restrict__ real, int R)
 {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     const size_t total = (size_t)nxh * nq * nslot * ny;
     if (i >= total) return;
     size_t r = i;
-    const int ky = r % ny; r /= ny;
+    const int L = ny / R;
+    const int sk = r % L; r /= L;
     const int s = r % nslot; r /= nslot;
     const int q = r % nq; r /= nq;
-    const int kx = (int)r;
+    const int kx = (int)(r % nxh), ky = R * sk + (int)(r / nxh);
     const size_t plane = (size_t)slot2c[s] + 9 * (size_t)real[q];
     const C2<double> v = TC[plane * nxh * ny + (size_t)ky * nxh + kx];
     Tspec[i] = C2<T>{(T)v.x, (T)v.y};
@@ -295,7 +298,7 @@ int Engine<T>::set_tensor_planes(const double* d_real, bool toeplitz)
     const size_t total = (size_t)nxh * nq * nslot * ny;
     RCHK(Tspec.alloc(total));
     hipLaunchKernelGGL(k_tensor_pack<T>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, c->stream, TC.p,
-                       Tspec.p, ny, nxh, nq, nslot, slot2c.p, d_real_of.p);
+                       Tspec.p, ny, nxh, nq, nslot, slot2c.p, d_real_of.p, subR);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(c->stream));
     toep = toeplitz;
