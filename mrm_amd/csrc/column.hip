@@ -158,9 +158,10 @@ template <typename T>
 template <int MB> void Engine<T>::launch_col_sym(int nb8)
 {
     const DemagOps<T> o = ops();
-    const dim3 g(nb8, 1, btab ? (unsigned)bn : 1u), b(col_threads);
+    const int th = col_th();
+    const dim3 g(nb8, 1, btab ? (unsigned)bn : 1u), b(th);
     if (pre) {
-        if (col_threads > 512)
+        if (th > 512)
             hipLaunchKernelGGL((k_col<T, MB, true, true, false, true, false, true>), g, b, lds_col, c->stream,
                                COL_ARGS);
         else
@@ -171,7 +172,7 @@ template <int MB> void Engine<T>::launch_col_sym(int nb8)
             hipLaunchKernelGGL((k_col<T, MB, true, true, false, false, true>), g, b, lds_col, c->stream, COL_ARGS);
         else
             hipLaunchKernelGGL((k_col<T, MB, true, false, false, false, true>), g, b, lds_col, c->stream, COL_ARGS);
-    } else if (col_threads > 512) {
+    } else if (th > 512) {
         if (tl)
             hipLaunchKernelGGL((k_col<T, MB, true, true, false, true>), g, b, lds_col, c->stream, COL_ARGS);
         else

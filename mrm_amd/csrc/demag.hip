@@ -631,7 +631,7 @@ int Engine<T>::launch_class(int cls)
             if (split && colp) return launch_colp();
         if (split) return set_err(MRMG_ERR_STATE, "the split path has no fused column kernel");
         const int nb8 = (nxh * kg + 7) / 8 * 8;
-        if (nslot == 6) LAUNCH_E(maxb_col, launch_col_sym, nb8);
+        if (nslot == 6) LAUNCH_E(col_th() > 512 ? maxb_big : maxb_col, launch_col_sym, nb8);
         else if (col_threads > 512) return set_err(MRMG_ERR_STATE, "col_threads 1024 needs the 6-slot tensor");
         else LAUNCH_E(maxb_col, launch_col_gen, nb8);
         break;

@@ -318,6 +318,8 @@ struct Engine : EngineBase {
     // launch shapes (mrmg_tune): threads of the row and column workgroups, observation-layer
     // groups per column workgroup, lanes per grain in the grain kernels
     int row_threads = 128, col_threads = 512, kg = 1, lpg = 8;
+    bool col_set = false;   // col_threads was asked for
+    int maxb_big = -1;      // elements per lane of the column kernel at 1024 threads
     bool lpg_set = false;   // lanes_per_grain was tuned: build() leaves it
     // split column path (column-contiguous spectra): rows per row workgroup, columns per
     // column workgroup, and whether it is in use (forced by col_path or by the grid size)
@@ -471,10 +473,11 @@ struct Engine : EngineBase {
                            nl);
         split = !fused_ok;
         if (split) RCHK(choose_split());
-        // long rows run fastest with the widest row workgroups (measured at 2048 points)
-        // and so do the split transform's row kernels (512x4096x4 FP64: 122 / 126 us with 256
-        // threads against 135 / 151 with 128)
-        if (nx >= 1024 || (subR > 1 && TYr_eff() * nx >= 4096)) row_threads = 256;
+        // 256 threads a row workgroup: a field's r2c / c2r of 256x256x4 FP64 9.6 / 9.6 us against
+        // 10.4 / 10.6 with 128, of 450x405x3 FP32 14.8 / 15.1 against 20.1 / 20.1, of 512x4096x4
+        // FP64 (split transform) 122 / 126 against 135 / 151.  The transposing kernels' shorter
+        // rows have the work for 128 only (512x4096x4 FP32: 58 / 55 against 57 / 59)
+        row_threads = !split || nx >= 1024 || (subR > 1 && TYr_eff() * nx >= 4096) ? 256 : 128;
         RCHK(shapes());
         RCHK(lds_attr());
         RCHK(S1.alloc((size_t)nl * 3 * ny * nxh));
@@ -594,6 +597,7 @@ struct Engine : EngineBase {
             if (split) return MRMG_OK;
         }
         maxb_row = pick_e(3, c->px, row_threads);
+        maxb_big = pick_e(3 * nl, c->py, 1024);
         const int ncw = col_threads / 64;
         maxb_col = tl && wv ? pick_e((3 * nl + ncw - 1) / ncw, c->py, 64) : pick_e(3 * nl, c->py, col_threads);
         if (maxb_row < 0 || maxb_col < 0)
@@ -623,6 +627,7 @@ struct Engine : EngineBase {
                 return set_err(MRMG_ERR_UNSUPPORTED, "col_threads 1024 needs the symmetric (6-slot) tensor");
             old = col_threads; col_threads = v;
             if (shapes() != MRMG_OK) { col_threads = old; return shapes(), MRMG_ERR_UNSUPPORTED; }
+            col_set = true;
         } else if (k == "col_groups") {
             if (v < 1 || v > c->nl) return set_err(MRMG_ERR_ARG, "col_groups must be in 1..n_lay");
             old = kg; kg = v;
@@ -698,6 +703,19 @@ struct Engine : EngineBase {
         return MRMG_OK;
     }
 
+    // Threads of the fused column kernel's workgroup.  Unless they were asked for, 1024 where
+    // the product has more than one item a thread at 512 (its tensor loads, a chain of n_lay/2
+    // round trips an item, are the longest part) and there is about one workgroup a CU, so that
+    // no other workgroup hides them: 21.3 us against 22.8 at 256x256x4 FP64, 29.7 against 32.3
+    // at 450x405x3 FP32, but 33 against 24 at 512x512x2 (257 workgroups) and 18.6 against 13.4
+    // at 512x256x1 (one item a thread of 256).
+    // Only where the 1024-thread kernel is built: one context, 6 slots, no wave-local FFTs.
+    int col_th() const
+    {
+        const int per = (c->nl + kg - 1) / kg;
+        const bool fits = !btab && !wv && !pre && nslot == 6 && maxb_big > 0 && maxb_big <= 16 && per * c->fy <= 2048;
+        return !col_set && fits && per * c->fy > 512 && c->nxh * kg <= 256 ? 1024 : col_threads;
+    }
     template <int MB> int lds_attr_mb();
     template <int MB> int lds_attr_col();
     template <int MB> int lds_attr_split();
