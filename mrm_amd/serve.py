@@ -70,7 +70,7 @@ def footprint_estimate(med, precision):
     tensor = 9 * nl * nl * kc * 2 * P
     spectra = 2 * 3 * nl * kc * 2 * P
     grains = 640 * G + 3 * P * G
-    per_cell = 4 * cells + 52 * cells
+    per_cell = 4 * cells + 44 * cells      # five ints of run lists and three FP64 run sums
     exchange = 12 * E + 4 * (G + 1)
     noise = 16 * 3 * 8 * G
     return tensor + spectra + grains + per_cell + exchange + noise + (2 << 20)

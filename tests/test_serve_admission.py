@@ -5,6 +5,7 @@ least recently used first, when a new request does not fit.  A stand-in batched 
 records which contexts it was given: a context is never in two batches at once, and a
 batch holds contexts of one key only."""
 import threading
+from types import SimpleNamespace
 
 import numpy as np
 
@@ -141,3 +142,12 @@ def test_pooled_contexts_are_counted(monkeypatch):
     assert len(dev.live) <= 1
     srv.close()
     assert not dev.live
+
+
+def test_estimate_counts_what_a_cell_adds():
+    """A request whose bytes fit is not turned away for bytes that no context holds: a cell
+    adds its entry of the grain map (4), and as a run of its own a place in the five run
+    lists (20) and its three FP64 run sums (24)."""
+    def est(cells):
+        return serve.footprint_estimate(SimpleNamespace(nx=64, ny=64, n_lay=1, G=100, cells=cells, layers=[]), 1)
+    assert est(3000) - est(1000) == 2000 * (4 + 5 * 4 + 3 * 8)
