@@ -114,7 +114,7 @@ struct RunsAhead {
 };
 
 // The cell field of the same rows, summed over each run (in x order, in FP64) into
-// Hr[c][run] (c = c0+ci), with the layout of runs_to_lds.
+// Hr[c] (c = c0+ci), with the layout of runs_to_lds.
 template <typename T, int NC, int RU>
 __device__ __forceinline__ void lds_to_runs(const RowRuns& R, RunsAhead<RU>& A, double* __restrict__ Hr, int c0,
                                             int nrows, int np, int nx, const T* re, const T* im, const int* roff)
@@ -123,6 +123,9 @@ __device__ __forceinline__ void lds_to_runs(const RowRuns& R, RunsAhead<RU>& A, 
     int yy = 0;   // increasing q: the row index only moves forward
     for (int qb = A.q0 + tid; qb < A.q1; qb += RU * nt) {
         if (qb != A.q0 + tid) A.fetch(R, qb, nt);
+        int to[RU];   // where the sums go: loaded here, not held across the FFT (4 to 8 registers)
+#pragma unroll
+        for (int u = 0; u < RU; u++) to[u] = R.perm && qb + u * nt < A.q1 ? R.perm[qb + u * nt] : qb + u * nt;
 #pragma unroll
         for (int u = 0; u < RU; u++) {
             const int q = qb + u * nt;
@@ -143,7 +146,7 @@ __device__ __forceinline__ void lds_to_runs(const RowRuns& R, RunsAhead<RU>& A, 
 #pragma unroll
                     for (int j = 0; j < MRMG_UF; j++) s += (double)(t + j < len ? a[j] : (T)0);
                 }
-                Hr[(size_t)(c0 + ci) * R.nruns + q] = s;
+                Hr[(size_t)(c0 + ci) * R.nruns + to[u]] = s;
             }
         }
     }

@@ -285,10 +285,12 @@ struct Engine : EngineBase {
     std::vector<int> off;
     // grain data
     DBuf<int> layer_of, gc_off, cell2grain;
-    // runs (RowRuns): grain by grain (run_off per grain, run_geo, run_row, run_q) and row by
-    // row (rrow_off per layer row, rrm_geo, rrm_grain)
-    DBuf<int> run_off, run_geo, run_row, run_q, rrow_off, rrm_geo, rrm_grain;
+    // runs (RowRuns): grain by grain (run_off per grain, run_geo, run_row) and row by row
+    // (rrow_off per layer row, rrm_geo, rrm_grain); run_map leads from the order that the run
+    // sums are not stored in to the one that they are (by_grain)
+    DBuf<int> run_off, run_geo, run_row, run_map, rrow_off, rrm_geo, rrm_grain;
     int nruns = 0;
+    bool by_grain = false;
     DBuf<int> x_off, x_nb;
     DBuf<S> x_w;
     DBuf<S> ms, msf, ms_scale, alpha_scale, hk_scale, hk1, hk2, uni, cub, happ, sigma, sigma_llb, vol;
@@ -409,7 +411,7 @@ struct Engine : EngineBase {
         size_t b = 0;
         b += layer_of.bytes() + gc_off.bytes() + cell2grain.bytes();
         b += run_off.bytes() + run_geo.bytes() + run_row.bytes() + rrow_off.bytes() + rrm_geo.bytes() + rrm_grain.bytes() +
-             run_q.bytes() + Mg.bytes() + Hr.bytes();
+             run_map.bytes() + Mg.bytes() + Hr.bytes();
         b += x_off.bytes() + x_nb.bytes() + x_w.bytes();
         b += ms.bytes() + msf.bytes() + ms_scale.bytes() + alpha_scale.bytes() + hk_scale.bytes() + hk1.bytes() +
              hk2.bytes() + uni.bytes() + cub.bytes() + happ.bytes() + sigma.bytes() + sigma_llb.bytes() + vol.bytes() +
@@ -637,6 +639,7 @@ struct Engine : EngineBase {
                 return set_err(MRMG_ERR_ARG, "lanes_per_grain must be 1, 2, 4, 8 or 16");
             lpg = v;
             lpg_set = true;
+            if (nruns > 0) RCHK(order_sums());
         } else if (k == "col_path") {
             if (v < 0 || v > 3)
                 return set_err(MRMG_ERR_ARG, "col_path must be 0 (fused), 1 (split), 2 (fused, column-contiguous) or 3 "
@@ -912,7 +915,8 @@ struct Engine : EngineBase {
                 rowoff[(size_t)layer[g] * ny + row[r] + 1]++;
             }
         for (size_t i = 1; i < rowoff.size(); i++) rowoff[i] += rowoff[i - 1];
-        std::vector<int> cur(rowoff.begin(), rowoff.end() - 1), rgeo(nruns), rgrain(nruns), rq(nruns);
+        by_grain = sums_by_grain(lpg);
+        std::vector<int> cur(rowoff.begin(), rowoff.end() - 1), rgeo(nruns), rgrain(nruns), map(nruns);
         std::vector<char> seen((size_t)nl * P, 0);
         for (int r = 0; r < nruns; r++) {
             const int g = grain_of[r];
@@ -926,20 +930,41 @@ struct Engine : EngineBase {
             const int q = cur[rw]++;
             rgeo[q] = geo[r];
             rgrain[q] = g;
-            rq[r] = q;
+            if (by_grain) map[q] = r;
+            else map[r] = q;
             row[r] |= layer[g] << RUN_LAYER_SHIFT;
         }
         geo.push_back(0);   // no array is empty
         row.push_back(0);
-        rgeo.push_back(0); rgrain.push_back(0); rq.push_back(0);
+        rgeo.push_back(0); rgrain.push_back(0); map.push_back(0);
         RCHK(run_off.upload(roff.data(), roff.size(), c->stream));
         RCHK(run_geo.upload(geo.data(), geo.size(), c->stream));
         RCHK(run_row.upload(row.data(), row.size(), c->stream));
         RCHK(rrow_off.upload(rowoff.data(), rowoff.size(), c->stream));
         RCHK(rrm_geo.upload(rgeo.data(), rgeo.size(), c->stream));
         RCHK(rrm_grain.upload(rgrain.data(), rgrain.size(), c->stream));
-        RCHK(run_q.upload(rq.data(), rq.size(), c->stream));
+        RCHK(run_map.upload(map.data(), map.size(), c->stream));
         HIPCHK(hipStreamSynchronize(c->stream));   // the host vectors go out of scope
+        return MRMG_OK;
+    }
+
+    // The order of the run sums.  The lanes of a grain (grain_sums_lanes) load its sums with
+    // their first loads when they are in its own runs' order; a wave that stages 64 grains'
+    // runs has the row order's index loads in flight together, and there the row kernels'
+    // consecutive stores count.
+    static bool sums_by_grain(int lanes) { return lanes > 1; }
+    // the map for the current lanes: its inverse, where the order changes (the sums themselves
+    // are rewritten before they are read)
+    int order_sums()
+    {
+        if (sums_by_grain(lpg) == by_grain) return MRMG_OK;
+        std::vector<int> a(nruns), b(nruns);
+        HIPCHK(hipMemcpyAsync(a.data(), run_map.p, sizeof(int) * nruns, hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(hipStreamSynchronize(c->stream));
+        for (int i = 0; i < nruns; i++) b[a[i]] = i;
+        HIPCHK(hipMemcpyAsync(run_map.p, b.data(), sizeof(int) * nruns, hipMemcpyHostToDevice, c->stream));
+        HIPCHK(hipStreamSynchronize(c->stream));
+        by_grain = !by_grain;
         return MRMG_OK;
     }
 
@@ -947,6 +972,7 @@ struct Engine : EngineBase {
     {
         RowRuns R;
         R.row_off = rrow_off.p; R.geo = rrm_geo.p; R.grain = rrm_grain.p; R.nruns = nruns;
+        R.perm = by_grain ? run_map.p : nullptr;
         return R;
     }
 
@@ -1094,7 +1120,7 @@ struct Engine : EngineBase {
         d.ms = ms.p; d.msf = msf.p; d.ms_scale = ms_scale.p; d.alpha_scale = alpha_scale.p; d.hk_scale = hk_scale.p;
         d.hk1 = hk1.p; d.hk2 = hk2.p; d.uni = uni.p; d.cub = cub.p; d.happ = has_happ ? happ.p : nullptr;
         d.sigma = sigma.p; d.vol = vol.p; d.gc_off = gc_off.p;
-        d.run_off = run_off.p; d.run_geo = run_geo.p; d.run_row = run_row.p; d.run_q = run_q.p; d.nruns = nruns;
+        d.run_off = run_off.p; d.run_geo = run_geo.p; d.run_row = run_row.p; d.run_q = by_grain ? nullptr : run_map.p; d.nruns = nruns;
         d.x_off = x_off.p; d.x_nb = x_nb.p; d.x_w = x_w.p;
         d.nl = c->nl;
         d.lp = lp.p;

@@ -314,28 +314,18 @@ __device__ __forceinline__ void grain_sums(const GrainData<T>& gd, const LayerPa
     }
 }
 
-// The sums of grain g by its own LPG lanes (4 and more lanes a grain, for media too small to
-// fill the chip with 64 grains a wave), which meet in a fixed butterfly: fewer steps one
-// after the other than through LDS (256x256x4, 15 692 grains, 8 lanes: 10.9 against 13.3 us).
-// LaneRound holds the index loads of a round, so that the first can be under way before the
-// workgroup's barrier.
-template <int LPG> struct LaneRound {
-    static constexpr int U = LPG <= 4 ? 2 : 1;   // runs and entries per lane and round
-    int r0, r1, x0, x1;
+// The index loads of one round of a grain's lanes: U runs and U exchange entries a lane.
+// Positions past the end load a valid entry, which is not added.
+template <int LPG, int U> struct LaneRound {
     int q[U], nb[U], geo[U], row[U];
     double w[U];
-    __device__ __forceinline__ void range(const int* run_off, const int* x_off, int g)
-    {
-        r0 = run_off[g]; r1 = run_off[g + 1];
-        x0 = x_off[g]; x1 = x_off[g + 1];
-    }
-    // positions past the end load a valid entry, which is not added
-    template <typename T> __device__ __forceinline__ void load(const GrainData<T>& gd, int b, bool src)
+    template <typename T>
+    __device__ __forceinline__ void load(const GrainData<T>& gd, int r0, int r1, int x0, int x1, int b, bool src)
     {
 #pragma unroll
         for (int u = 0; u < U; u++) {
             const int r = r0 + b + u * LPG, e = x0 + b + u * LPG, rc = r < r1 ? r : r0, ec = e < x1 ? e : x0;
-            q[u] = at32(gd.run_q, rc);
+            q[u] = gd.run_q ? at32(gd.run_q, rc) : rc;
             nb[u] = at32(gd.x_nb, ec);
             w[u] = at32(gd.x_w, ec);
             if (src) {
@@ -346,44 +336,45 @@ template <int LPG> struct LaneRound {
     }
 };
 
+// The sums of a grain (runs [r0, r1), exchange entries [x0, x1)) by its own LPG lanes (two and
+// more lanes a grain, for media too small to fill the chip with 64 grains a wave), which meet
+// in a fixed butterfly: fewer steps one after the other than through LDS (256x256x4, 15 692
+// grains, 8 lanes: 10.2 against 13.3 us).  A small medium's stage is a chain of dependent
+// loads and nothing else, so a layer without a source has a loop of its own, of two runs and
+// entries a lane and round: as one loop with the sources' branches, a round of one entry a
+// lane and 8 lanes, a second round was due for every ninth neighbour and a stage took 0.2 us
+// more (64x64x1), with 4 lanes 23.2 against 22.2 us (31 302 grains) and 59 against 48 (119 640).
 template <typename T, int LPG>
-__device__ __forceinline__ void grain_sums_lanes(const GrainData<T>& gd, const LayerParams* lp, int k, int lane,
-                                                 const T* __restrict__ mf, const double* __restrict__ Hr,
-                                                 bool temps_only, LaneRound<LPG>& I, GrainSums& S)
+__device__ __forceinline__ void grain_sums_lanes(const GrainData<T>& gd, const LayerParams* lp, int k, int fk, int tk,
+                                                 int lane, int r0, int r1, int x0, int x1, const T* __restrict__ mf,
+                                                 const double* __restrict__ Hr, bool temps_only, GrainSums& S)
 {
-    constexpr int U = LaneRound<LPG>::U;
     const int G = gd.G, nt = gd.n_temp;
-    const bool fsrc = gd.any_fsrc && !temps_only && lp[k].src[0].kind == MRMG_SRC_FIELD_TABLE;
-    const bool tsrc = nt > 0 && lp[k].src[1].kind != MRMG_SRC_NONE;
-    const bool tsg = tsrc && lp[k].src[1].kind == MRMG_SRC_TEMP_SG;
+    const bool fsrc = !temps_only && fk == MRMG_SRC_FIELD_TABLE;
+    const bool tsrc = nt > 0 && tk != MRMG_SRC_NONE, tsg = tsrc && tk == MRMG_SRC_TEMP_SG;
     const size_t NR = (size_t)gd.nruns;
     const T* __restrict__ msc = mf + (size_t)ST_MSC * G;
     double hd[3] = {0, 0, 0}, hx[3] = {0, 0, 0}, tt[2] = {0, 0}, hs[3] = {0, 0, 0};
-    const int nr = I.r1 - I.r0, nx = I.x1 - I.x0, n = temps_only || nr > nx ? nr : nx;
-    for (int b = lane; b < n; b += U * LPG) {
-        double hv[U][3], xv[U][4], tv[U][2];
-        if (!temps_only)
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-#pragma unroll
-                for (int c = 0; c < 3; c++) {
-                    hv[u][c] = Hr ? at32(Hr + c * NR, I.q[u]) : 0.0;
-                    xv[u][c] = at32(mf + (size_t)c * G, I.nb[u]);
-                }
-                xv[u][3] = at32(msc, I.nb[u]);
-            }
-        if (tsg)
+    const int nr = r1 - r0, nx = x1 - x0, n = temps_only || nr > nx ? nr : nx;
+    if (!fsrc && !tsrc) {
+        constexpr int U = 2;
+        for (int b = lane; !temps_only && b < n; b += U * LPG) {
+            LaneRound<LPG, U> I;
+            I.load(gd, r0, r1, x0, x1, b, false);
+            double hv[U][3], xv[U][4];
 #pragma unroll
             for (int u = 0; u < U; u++)
 #pragma unroll
-                for (int ts = 0; ts < 2; ts++)
-                    if (ts < nt)
-                        tv[u][ts] = sg_run(gd.ax, k, ts, I.geo[u] & 0xffff, I.geo[u] >> 16, I.row[u] & RUN_ROW_MASK);
+                for (int c = 0; c < 3; c++) hv[u][c] = Hr ? at32(Hr + c * NR, I.q[u]) : 0.0;
 #pragma unroll
-        for (int u = 0; u < U; u++) {
-            const bool hr = b + u * LPG < nr;
-            if (!temps_only) {
-                if (hr) {
+            for (int u = 0; u < U; u++) {
+#pragma unroll
+                for (int c = 0; c < 3; c++) xv[u][c] = at32(mf + (size_t)c * G, I.nb[u]);
+                xv[u][3] = at32(msc, I.nb[u]);
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                if (b + u * LPG < nr) {
 #pragma unroll
                     for (int c = 0; c < 3; c++) hd[c] += hv[u][c];
                 }
@@ -393,29 +384,67 @@ __device__ __forceinline__ void grain_sums_lanes(const GrainData<T>& gd, const L
                     for (int c = 0; c < 3; c++) hx[c] += wm * xv[u][c];
                 }
             }
-            if (tsg && hr) {
-                tt[0] += tv[u][0];
-                if (nt > 1) tt[1] += tv[u][1];
-            }
         }
-        if ((tsrc && !tsg) || fsrc)
+    } else {
+        constexpr int U = LPG <= 4 ? 2 : 1;
+        for (int b = lane; b < n; b += U * LPG) {
+            LaneRound<LPG, U> I;
+            I.load(gd, r0, r1, x0, x1, b, true);
+            double hv[U][3], xv[U][4], tv[U][2];
+            if (!temps_only)
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+#pragma unroll
+                    for (int c = 0; c < 3; c++) {
+                        hv[u][c] = Hr ? at32(Hr + c * NR, I.q[u]) : 0.0;
+                        xv[u][c] = at32(mf + (size_t)c * G, I.nb[u]);
+                    }
+                    xv[u][3] = at32(msc, I.nb[u]);
+                }
+            if (tsg)
+#pragma unroll
+                for (int u = 0; u < U; u++)
+#pragma unroll
+                    for (int ts = 0; ts < 2; ts++)
+                        if (ts < nt)
+                            tv[u][ts] = sg_run(gd.ax, k, ts, I.geo[u] & 0xffff, I.geo[u] >> 16, I.row[u] & RUN_ROW_MASK);
 #pragma unroll
             for (int u = 0; u < U; u++) {
-                if (b + u * LPG >= nr) break;
-                const int i0 = I.geo[u] & 0xffff, len = I.geo[u] >> 16, j = I.row[u] & RUN_ROW_MASK;
-                double v[3];
-                if (tsrc && !tsg)
-                    for (int ts = 0; ts < nt; ts++) {
-                        table_run<1>(gd.ax, lp[k].src[1], k, 1, ts, i0, len, j, v);
-                        tt[ts] += v[0];
-                    }
-                if (fsrc) {
-                    table_run<3>(gd.ax, lp[k].src[0], k, 0, 0, i0, len, j, v);
+                const bool hr = b + u * LPG < nr;
+                if (!temps_only) {
+                    if (hr) {
 #pragma unroll
-                    for (int c = 0; c < 3; c++) hs[c] += v[c];
+                        for (int c = 0; c < 3; c++) hd[c] += hv[u][c];
+                    }
+                    if (b + u * LPG < nx) {
+                        const double wm = I.w[u] * xv[u][3];
+#pragma unroll
+                        for (int c = 0; c < 3; c++) hx[c] += wm * xv[u][c];
+                    }
+                }
+                if (tsg && hr) {
+                    tt[0] += tv[u][0];
+                    if (nt > 1) tt[1] += tv[u][1];
                 }
             }
-        if (b + U * LPG < n) I.load(gd, b + U * LPG, nt > 0 || gd.any_fsrc);
+            if ((tsrc && !tsg) || fsrc)
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    if (b + u * LPG >= nr) break;
+                    const int i0 = I.geo[u] & 0xffff, len = I.geo[u] >> 16, j = I.row[u] & RUN_ROW_MASK;
+                    double v[3];
+                    if (tsrc && !tsg)
+                        for (int ts = 0; ts < nt; ts++) {
+                            table_run<1>(gd.ax, lp[k].src[1], k, 1, ts, i0, len, j, v);
+                            tt[ts] += v[0];
+                        }
+                    if (fsrc) {
+                        table_run<3>(gd.ax, lp[k].src[0], k, 0, 0, i0, len, j, v);
+#pragma unroll
+                        for (int c = 0; c < 3; c++) hs[c] += v[c];
+                    }
+                }
+        }
     }
 #pragma unroll
     for (int c = 0; c < 3; c++) {
@@ -431,11 +460,11 @@ __device__ __forceinline__ void grain_sums_lanes(const GrainData<T>& gd, const L
 // evaluation and at the next evaluation from the layer's temperature source
 // (field.f90:545-556), unchanged without one
 template <typename T>
-__device__ __forceinline__ void field_at(const GrainData<T>& gd, const LayerParams& L, int g, const GrainSums& S,
-                                         bool demag, double t, const T* m, T* h, double* tout, const GrainPre<T>& P)
+__device__ __forceinline__ void field_at(const GrainData<T>& gd, const LayerParams& L, bool fsrc, bool tsrc, int g,
+                                         const GrainSums& S, bool demag, double t, const T* m, T* h, double* tout,
+                                         const GrainPre<T>& P)
 {
     const int G = gd.G;
-    const bool fsrc = L.src[0].kind == MRMG_SRC_FIELD_TABLE, tsrc = L.src[1].kind != MRMG_SRC_NONE;
     const T hk_s = P.hk_s, hk1 = P.hk1, hk2 = P.hk2;
     const T u[3] = {P.u[0], P.u[1], P.u[2]};
     T happ[3] = {P.happ[0], P.happ[1], P.happ[2]};
@@ -920,9 +949,9 @@ __device__ __forceinline__ void grain_body(const GrainData<T>& gd, T* __restrict
     const int bl = xcd_remap(blockIdx.x, gridDim.x);
     if (bl >= nblk) return;
     const int G = gd.G;
-    // LPG <= 2: lane l < 64 / LPG of a wave has the wave's grain l and the other lanes only
-    // help to load; else every lane of a grain computes its results and its first one stores
-    constexpr bool WAVE = LPG <= 2;
+    // LPG 1: lane l of a wave has the wave's grain l, and the lanes load for each other; else
+    // every lane of a grain computes its results and its first one stores
+    constexpr bool WAVE = LPG == 1;
     constexpr int NGW = 64 / LPG;
     const int wv = (int)threadIdx.x >> 6, ln = (int)threadIdx.x & 63;
     const int gw0 = __builtin_amdgcn_readfirstlane(bl * (256 / LPG) + wv * NGW);
@@ -956,15 +985,17 @@ __device__ __forceinline__ void grain_body(const GrainData<T>& gd, T* __restrict
         g_as = gd.alpha_scale[g];
         g_temp = gd.temp[g];
     };
-    LaneRound<WAVE ? 8 : LPG> I;
+    int r0 = 0, r1 = 0, x0 = 0, x1 = 0;
     if constexpr (!WAVE) {
-        I.range(gd.run_off, gd.x_off, g);
+        r0 = gd.run_off[g]; r1 = gd.run_off[g + 1];
+        x0 = gd.x_off[g]; x1 = gd.x_off[g + 1];
         if constexpr (LPG >= 8) load();
-        if (MODE != GM_PUSH1 || gd.n_temp > 0) I.load(gd, ln % LPG, gd.n_temp > 0 || gd.any_fsrc);
     }
     {
         // the layers' parameters into LDS: those this workgroup's grains lie in, or, where a
-        // launch is a few workgroups and only its latency counts, all in one sweep
+        // launch is a few workgroups and only its latency counts, all in one sweep.  (The
+        // workgroup's 256 threads as a constant: blockDim.x is a vector load here, and its wait
+        // one for every load before it, 0.2 to 0.4 us a stage.)
         typedef unsigned long long u64;
         constexpr int nw = (int)(sizeof(LayerParams) / sizeof(u64));
         const u64* src = reinterpret_cast<const u64*>(gd.lp);
@@ -973,15 +1004,17 @@ __device__ __forceinline__ void grain_body(const GrainData<T>& gd, T* __restrict
             const int b0 = bl * (256 / LPG), b1 = b0 + 256 / LPG;
             for (int q = 0; q < gd.nl; q++)
                 if (gd.loff[q] < b1 && gd.loff[q + 1] > b0)
-                    for (int i = threadIdx.x; i < nw; i += blockDim.x) dst[q * nw + i] = src[q * nw + i];
+                    for (int i = threadIdx.x; i < nw; i += 256) dst[q * nw + i] = src[q * nw + i];
         } else {
-            for (int i = threadIdx.x; i < gd.nl * nw; i += blockDim.x) dst[i] = src[i];
+            for (int i = threadIdx.x; i < gd.nl * nw; i += 256) dst[i] = src[i];
         }
     }
     if (a.diag)
-        for (int i = threadIdx.x; i < DIAG_STRIDE; i += blockDim.x) red[i] = 0.0;
+        for (int i = threadIdx.x; i < DIAG_STRIDE; i += 256) red[i] = 0.0;
     __syncthreads();
     const LayerParams& L = slp[k];
+    const int fk = L.src[0].kind, tk = L.src[1].kind;   // read once: each LDS read is waited for in turn
+    const bool fsrc = fk == MRMG_SRC_FIELD_TABLE, tsrc = tk != MRMG_SRC_NONE;
     T h[3] = {0, 0, 0};
     double tev[2] = {0, 0};   // grain temperature now and at the next evaluation (moving sources)
     GrainSums S;
@@ -990,16 +1023,16 @@ __device__ __forceinline__ void grain_body(const GrainData<T>& gd, T* __restrict
             grain_sums<T, LPG>(gd, slp, gw0, ngw, mf, Hr, MODE == GM_PUSH1,
                                gval + wv * GrainShape<LPG>::doubles(gd.n_temp), S);
         else
-            grain_sums_lanes<T, LPG>(gd, slp, k, ln % LPG, mf, Hr, MODE == GM_PUSH1, I, S);
+            grain_sums_lanes<T, LPG>(gd, slp, k, fk, tk, ln % LPG, r0, r1, x0, x1, mf, Hr, MODE == GM_PUSH1, S);
     }
     if (act) {
     if constexpr (LPG < 8) load();
     if (MODE != GM_PUSH1) {
-        field_at<T>(gd, L, g, S, Hr != nullptr, a.clk ? a.clk[0] + a.t : a.t, mfield, h, tev, P);
+        field_at<T>(gd, L, fsrc, tsrc, g, S, Hr != nullptr, a.clk ? a.clk[0] + a.t : a.t, mfield, h, tev, P);
     } else {
 #pragma unroll
         for (int c = 0; c < 3; c++) h[c] = hout[(size_t)c * G + g];
-        if (L.src[1].kind != MRMG_SRC_NONE) {
+        if (tsrc) {
             const double dc = (double)P.cells;
             tev[0] = S.t[0] / dc + g_temp;
             if (gd.n_temp > 1) tev[1] = S.t[1] / dc + g_temp;
@@ -1009,7 +1042,6 @@ __device__ __forceinline__ void grain_body(const GrainData<T>& gd, T* __restrict
     T fsc = 0;   // Ms * ms_scale of the new state: the cell magnetisation factor
     {
         // the grain temperature of this evaluation and the next one
-        const bool tsrc = L.src[1].kind != MRMG_SRC_NONE;
         double Tev = g_temp, Tnx = Tev;
         if (tsrc) {
             Tnx = tev[1];
@@ -1174,7 +1206,7 @@ __device__ __forceinline__ void grain_body(const GrainData<T>& gd, T* __restrict
     }
     if (a.diag) {
         __syncthreads();
-        for (int i = threadIdx.x; i < DIAG_STRIDE; i += blockDim.x) diag_part[(size_t)bl * DIAG_STRIDE + i] = red[i];
+        for (int i = threadIdx.x; i < DIAG_STRIDE; i += 256) diag_part[(size_t)bl * DIAG_STRIDE + i] = red[i];
     }
 }
 
@@ -1446,7 +1478,7 @@ template <int MODE, int LPG> int Engine<T>::launch_grain(const StepArgs& a, S* m
     const size_t threads = (size_t)G * LPG;
     const unsigned nb8 = (unsigned)(((threads + 255) / 256 + 7) / 8 * 8);
     hipLaunchKernelGGL((k_grain<S, MODE, LPG, T>), dim3(nb8), dim3(256),
-                       LPG <= 2 ? 4 * sizeof(double) * GrainShape<LPG>::doubles(n_temp) : 0, c->stream,
+                       LPG == 1 ? 4 * sizeof(double) * GrainShape<LPG>::doubles(n_temp) : 0, c->stream,
                        gdata(), ma.p, mb.p, dm.p, hthm.p, h.p, demag_on() ? Hr.p : nullptr,
                        demag_on() ? Mg.p : nullptr, a, diag_part.p, mout);
     HIPCHK(hipGetLastError());

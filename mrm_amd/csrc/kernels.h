@@ -136,12 +136,16 @@ __host__ __device__ inline size_t tensor_block(int kx, int ko, int ks, int nl, i
 // data.f90:344-353) and write the cell field's sums over them, which the grain kernels add
 // up (get_magnetostatic, field.f90:463-468); no cell array goes to memory.  Runs are
 // numbered grain by grain (each grain's runs contiguous, in the order of its cells) and
-// listed a second time row by row for the row kernels, which write their sums in that order
-// (consecutive lanes, consecutive runs); the grain kernels read them through run_q.
+// listed a second time row by row for the row kernels.  The sums are stored in one of the two
+// orders (Engine::sums_by_grain): row by row, as the row kernels come to them (consecutive
+// lanes, consecutive runs), and the grain kernels read them through run_q; or grain by grain,
+// the row kernels writing them through perm, and a grain's sums are its own runs', with no
+// index to be loaded first.
 struct RowRuns {
     const int* row_off;   // [nl*ny + 1]: the runs of row (k, y) are [row_off[k*ny + y], row_off[k*ny + y + 1])
     const int* geo;       // row by row: first x | length << 16
     const int* grain;     // row by row: global grain
+    const int* perm;      // row by row: the run's grain-by-grain number, or null: sums row by row
     int nruns;
 };
 // the row and the layer of a run in one word (GrainData::run_row): no row FFT of 2^24 rows
@@ -158,7 +162,7 @@ template <typename T> struct DemagOps {
     C2<T>* S2;              // spectra of H
     const C2<T>* Tspec;     // tensor spectra
     T* Hcell;               // cell field (mrmg_demag_field only)
-    double* Hr;             // [3][nruns] run sums of the cell field, row by row
+    double* Hr;             // [3][nruns] run sums of the cell field
     RowRuns R;
     int G, pad_;
 };
@@ -205,7 +209,7 @@ template <typename T> struct GrainData {
     // wider loads cost more than they saved, 179 against 161 us in the 2048x2048x8 write)
     const int* run_geo;   //   first x | length << 16
     const int* run_row;   //   row y within the grain's layer | layer << RUN_LAYER_SHIFT
-    const int* run_q;     //   the run's number in the row-by-row order (the run sums' order)
+    const int* run_q;     //   the run's number in the row-by-row order, or null: sums grain by grain
     int nruns;
     // exchange CSR, per grain the intralayer entries, then those to the layer above, then
     // to the layer below, and one spare entry at the end

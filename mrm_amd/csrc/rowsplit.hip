@@ -99,13 +99,14 @@ __device__ __forceinline__ void split_lds_to_runs(const RowRuns& R, const SplitR
     const int nt = (int)blockDim.x, n = S.runs();
     int last = 0;
     for (int tb = (int)threadIdx.x; tb < n; tb += RU * nt) {
-        int geo[RU], row[RU], q[RU];
+        int geo[RU], row[RU], to[RU];
 #pragma unroll
         for (int u = 0; u < RU; u++)
             if (tb + u * nt < n) {
                 last = row[u] = S.row_of(tb + u * nt, last);
-                q[u] = S.base[row[u]] + tb + u * nt;
-                geo[u] = R.geo[q[u]];
+                const int q = S.base[row[u]] + tb + u * nt;
+                geo[u] = R.geo[q];
+                to[u] = R.perm ? R.perm[q] : q;
             }
 #pragma unroll
         for (int u = 0; u < RU; u++) {
@@ -121,7 +122,7 @@ __device__ __forceinline__ void split_lds_to_runs(const RowRuns& R, const SplitR
 #pragma unroll
                 for (int j = 0; j < MRMG_UF; j++) s += (double)(t + j < len ? a[j] : (T)0);
             }
-            Hr[q[u]] = s;
+            Hr[to[u]] = s;
         }
     }
 }
