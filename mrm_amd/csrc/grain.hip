@@ -343,7 +343,8 @@ template <int LPG, int U> struct LaneRound {
 // loads and nothing else, so a layer without a source has a loop of its own, of two runs and
 // entries a lane and round: as one loop with the sources' branches, a round of one entry a
 // lane and 8 lanes, a second round was due for every ninth neighbour and a stage took 0.2 us
-// more (64x64x1), with 4 lanes 23.2 against 22.2 us (31 302 grains) and 59 against 48 (119 640).
+// more (64x64x1: 8.65 now), and two stages with 4 lanes took 23.2 against 21.2 us (31 302
+// grains) and 59 against 48 (119 640).
 template <typename T, int LPG>
 __device__ __forceinline__ void grain_sums_lanes(const GrainData<T>& gd, const LayerParams* lp, int k, int fk, int tk,
                                                  int lane, int r0, int r1, int x0, int x1, const T* __restrict__ mf,
@@ -966,8 +967,9 @@ __device__ __forceinline__ void grain_body(const GrainData<T>& gd, T* __restrict
     const T* mf = (MODE == GM_HEUN2 || MODE == GM_ROT2) ? mb : ma;
     // the grain's state and constants: with 8 and more lanes a grain issued first, so that
     // they overlap the sums' loads; with fewer loaded after the sums, since held across them
-    // they would cost waves in flight (250 registers against 162 with one lane, 264 against
-    // 154 with four: 30.9 against 22.0 us at 32 680 grains)
+    // they would cost waves in flight (two stages with four lanes: 48 us against 54 at 119 640
+    // grains and 47 against 55 at 36 416 under a moving field table, but 22.2 against 20.5 at
+    // 31 302)
     GrainPre<T> P;
     T mfield[3], mi[3], msc, g_ms, g_msf, g_vol, g_sig, g_as, dmv[3] = {0, 0, 0}, thv[3] = {0, 0, 0};
     double g_temp;
