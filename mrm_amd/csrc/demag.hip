@@ -617,7 +617,8 @@ int Engine<T>::launch_class(int cls)
     // out (RowSplit), nxh of fy values unless the transform is split
     const int ny = c->ny, fy = vL(), nl = c->nl, nxh = vnx();
     const unsigned z = btab ? (unsigned)bn : 1u;
-    const dim3 grow((ny + 1) / 2, nl, z), growT(rowT_blocks(), 1, z), blk(row_threads), b256(256);
+    const int rth = row_th(), mbr = rth == row_threads ? maxb_row : pick_e(3, c->px, rth);
+    const dim3 grow((ny + 1) / 2, nl, z), growT(rowT_blocks(), 1, z), blk(rth), b256(256);
     const int ncols = 3 * nl * nxh;
     const dim3 gcol((ncols + CBc - 1) / CBc, 1, z);
     if (btab && (wv || cells_out))
@@ -627,7 +628,7 @@ int Engine<T>::launch_class(int cls)
         if constexpr (sizeof(T) == 8)
             if (subR > 1) return launch_rowS(false, growT, blk);
         if (tl || split) LAUNCH_E(maxb_rowT, launch_rowT_fwd, growT, blk);
-        else LAUNCH_E(maxb_row, launch_row_fwd, grow, blk);
+        else LAUNCH_E(mbr, launch_row_fwd, grow, blk);
         break;
     case K_COL: {
         if constexpr (sizeof(T) == 8)
@@ -678,7 +679,7 @@ int Engine<T>::launch_class(int cls)
         if constexpr (sizeof(T) == 8)
             if (subR > 1) return launch_rowS(true, growT, blk);
         if (tl || split) LAUNCH_E(maxb_rowT, launch_rowT_inv, growT, blk);
-        else LAUNCH_E(maxb_row, launch_row_inv, grow, blk);
+        else LAUNCH_E(mbr, launch_row_inv, grow, blk);
         break;
     default:
         return set_err(MRMG_ERR_ARG, "not a demag kernel class");

@@ -320,6 +320,7 @@ struct Engine : EngineBase {
     // launch shapes (mrmg_tune): threads of the row and column workgroups, observation-layer
     // groups per column workgroup, lanes per grain in the grain kernels
     int row_threads = 128, col_threads = 512, kg = 1, lpg = 8;
+    int row_def = 128;      // the row threads that were not asked for (row_th)
     bool col_set = false;   // col_threads was asked for
     int maxb_big = -1;      // elements per lane of the column kernel at 1024 threads
     bool lpg_set = false;   // lanes_per_grain was tuned: build() leaves it
@@ -475,11 +476,15 @@ struct Engine : EngineBase {
                            nl);
         split = !fused_ok;
         if (split) RCHK(choose_split());
-        // 256 threads a row workgroup: a field's r2c / c2r of 256x256x4 FP64 9.6 / 9.6 us against
-        // 10.4 / 10.6 with 128, of 450x405x3 FP32 14.8 / 15.1 against 20.1 / 20.1, of 512x4096x4
-        // FP64 (split transform) 122 / 126 against 135 / 151.  The transposing kernels' shorter
-        // rows have the work for 128 only (512x4096x4 FP32: 58 / 55 against 57 / 59)
-        row_threads = !split || nx >= 1024 || (subR > 1 && TYr_eff() * nx >= 4096) ? 256 : 128;
+        // 256 threads a row workgroup: a field's r2c / c2r of 256x256x4 FP64 6.6 / 6.4 us against
+        // 7.2 / 6.8 with 128, of 450x405x3 FP32 11.9 / 11.7 against 15.2 / 15.8, of 512x4096x4
+        // FP64 (split transform) 122 / 126 against 135 / 151; of 96x96x2 FP32 6.0 / 6.6 against
+        // 6.3 / 6.7.  Three rows of 64 points are 192 elements, which leave a wave of 256 threads
+        // idle: 64x64x1 with 128 a step of 57.9 us against 58.3 (FP64) and 55.1 against 55.7.  On
+        // grids for the transposing kernels alone the shorter rows have the work for 128 only
+        // (512x4096x4 FP32: 58 / 55 against 57 / 59).  A full chip: row_th
+        row_def = split ? (nx >= 1024 || (subR > 1 && TYr_eff() * nx >= 4096) ? 256 : 128) : 3 * nx <= 256 ? 128 : 256;
+        row_threads = row_def;
         RCHK(shapes());
         RCHK(lds_attr());
         RCHK(S1.alloc((size_t)nl * 3 * ny * nxh));
@@ -706,6 +711,20 @@ struct Engine : EngineBase {
         return MRMG_OK;
     }
 
+    // Threads of the fused path's row workgroups.  A batch can have more of them than the chip
+    // holds at once with 256 threads (FP32 seven a CU, FP64 five, by their registers).  Then
+    // rows of up to 300 points take 128, unless the threads were asked for: a step of batches
+    // with 128 / 256, us, FP32 128x128x2 1024 workgroups 92 / 91, 1536 124 / 125, 2048
+    // 134 / 150, 4096 212 / 233; 288x128x2 1536 196 / 188, 2048 230 / 238; FP64 128x128x2 1024
+    // 115 / 114, 1536 137 / 153; 288x128x2 1024 188 / 176, 1536 233 / 241.  From 320 points on a
+    // thread of 128 has more than seven elements of the three rows, and 256 keep the lead or
+    // draw level (FP64 320x128x2, 2048 workgroups: 312 / 297; FP32 417 / 422 at 4096).
+    int row_th() const
+    {
+        const size_t wg = (size_t)(c->ny + 1) / 2 * c->nl * (btab ? bn : 1);
+        const bool full = wg > (sizeof(T) == 4 ? 7 : 5) * 256;
+        return full && row_threads == row_def && !split && !tl && c->fx <= 300 ? 128 : row_threads;
+    }
     // Threads of the fused column kernel's workgroup.  Unless they were asked for, 1024 where
     // the product has more than one item a thread at 512 (its tensor loads, a chain of n_lay/2
     // round trips an item, are the longest part) and there is about one workgroup a CU, so that
