@@ -393,7 +393,10 @@ int mrmg_tune(mrmg_ctx *ctx, const char *key, int value);
 /* The value of a tunable, or of the read-only key "tensor_offsets": 1 when the stored
  * tensor spectra are the 2 n_lay - 1 z-offset blocks (the tensor depends on the layer pair
  * only through ko - ks: equal thicknesses and spacings, no magnetic images above or
- * below), 0 when they are the n_lay^2 layer-pair blocks. */
+ * below), 0 when they are the n_lay^2 layer-pair blocks; or "col_split": where the column
+ * FFTs, the product and the inverse run as one kernel between row kernels that take a radix
+ * of the column transform (FP64, grids for the split path, up to 4 layers, z-offset tensor
+ * of 6 slots), that radix (1: none of it), else 0. */
 int mrmg_get_tune(mrmg_ctx *ctx, const char *key, int *value);
 /* Copies up to max entries; *n receives the number of kernel classes. */
 int mrmg_kernel_stats(mrmg_ctx *ctx, mrmg_kstat *out, int max, int *n);

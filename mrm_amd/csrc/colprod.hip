@@ -102,7 +102,7 @@ int Engine<double>::launch_colp()
 {
     const DemagOps<double> o = ops();
     const int z = btab ? bn : 1, L = vL(), th = colp_threads, e = pick_e(3 * c->nl, pcol, th);
-    if (e < 0 || e > 32 || nslot != 6 || !toep) return set_err(MRMG_ERR_STATE, "the one-kernel column path does not fit");
+    if (e < 0 || e > 32 || nslot != 6 || !one_fit) return set_err(MRMG_ERR_STATE, "the one-kernel column path does not fit");
 #define KCN(N)                                                                                                          \
     case N:                                                                                                             \
         return e > 16 ? launch_colp_nl<double, 32, N>(c->stream, z, th, lds_colp, o, btab, L, vnx(), pcol, twy.p)       \

@@ -335,8 +335,8 @@ struct Engine : EngineBase {
     int TYr = 8, CBc = 1, maxb_rowT = 4, maxb_colT = 4;
     // the split of the column transform (RowSplit): its radix, the media rows of a group; the
     // one-kernel column path (colprod.hip) and its launch shape
-    int subR = 1, subRm = 1, colp_threads = 256;
-    bool colp = false;
+    int subR = 1, subRm = 1, colp_threads = 256, ty_def = 8;   // ty_def: TYr before any row_block
+    bool colp = false, one_fit = true;                         // one_fit: choose_split's argument
     size_t lds_colp = 0;
     DBuf<C2<T>> tws;
     // FFT plans of the step's row and column transforms and their largest radix
@@ -435,6 +435,8 @@ struct Engine : EngineBase {
         if (!s->tensor_ok) return set_err(MRMG_ERR_STATE, "the source context has no tensor");
         HIPCHK(hipStreamSynchronize(s->c->stream));
         RCHK(set_slots(s->nslot == 6));
+        RCHK(fit_split(s->toep));
+        if (subR != s->subR) return set_err(MRMG_ERR_STATE, "the two contexts lay their columns out differently");
         RCHK(Tspec.alloc(s->Tspec.n));
         HIPCHK(hipMemcpyAsync(Tspec.p, s->Tspec.p, Tspec.bytes(), hipMemcpyDeviceToDevice, c->stream));
         HIPCHK(hipStreamSynchronize(c->stream));
@@ -475,7 +477,8 @@ struct Engine : EngineBase {
             return set_err(MRMG_ERR_UNSUPPORTED, "grid %dx%dx%d: a row or column FFT does not fit one workgroup", nx, ny,
                            nl);
         split = !fused_ok;
-        if (split) RCHK(choose_split());
+        ty_def = TYr;
+        if (split) RCHK(choose_split(true));   // again when the tensor is known (fit_split)
         // 256 threads a row workgroup: a field's r2c / c2r of 256x256x4 FP64 6.6 / 6.4 us against
         // 7.2 / 6.8 with 128, of 450x405x3 FP32 11.9 / 11.7 against 15.2 / 15.8, of 512x4096x4
         // FP64 (split transform) 122 / 126 against 135 / 151; of 96x96x2 FP32 6.0 / 6.6 against
@@ -483,8 +486,7 @@ struct Engine : EngineBase {
         // idle: 64x64x1 with 128 a step of 57.9 us against 58.3 (FP64) and 55.1 against 55.7.  On
         // grids for the transposing kernels alone the shorter rows have the work for 128 only
         // (512x4096x4 FP32: 58 / 55 against 57 / 59).  A full chip: row_th
-        row_def = split ? (nx >= 1024 || (subR > 1 && TYr_eff() * nx >= 4096) ? 256 : 128) : 3 * nx <= 256 ? 128 : 256;
-        row_threads = row_def;
+        row_threads = row_def = row_default();
         RCHK(shapes());
         RCHK(lds_attr());
         RCHK(S1.alloc((size_t)nl * 3 * ny * nxh));
@@ -509,14 +511,18 @@ struct Engine : EngineBase {
     // * the product's registers hold the layers (4);
     // * the row kernels' rows take at most 4096 transform elements (70 KB; 64 a thread with
     //   the fewest threads that can be asked for).
-    int choose_split()
+    // one: the tensor is one that the kernel takes (z-offset blocks of six slots).  Any other
+    // keeps the unsplit columns: over split ones its three kernels gained less in the columns
+    // than the rows lost (a step, us, unequal layers: 256x2048x4 rows 27 / 27 a field against
+    // 38 / 34, columns 52 against 48; open 64x384x3 129 against 142)
+    int choose_split(bool one)
     {
         const int nl = c->nl, fy = c->fy;
         subR = subRm = 1;
         colp = false;
-        if (sizeof(T) != 8 || nl > 4) return MRMG_OK;
-        for (int R = 8; R >= (c->open ? 2 : 1) && !colp; R /= 2) {
-            const int L = fy / R, rm = c->open ? R / 2 : R, ty = std::max(TYr, rm);
+        pcol = c->py;
+        for (int R = 8; R >= (c->open ? 2 : 1) && !colp && one && sizeof(T) == 8 && nl <= 4; R /= 2) {
+            const int L = fy / R, rm = c->open ? R / 2 : R, ty = std::max(ty_def, rm);
             FFTPlan q;
             if (fy % R != 0 || L < 256 || !factorize(L, q)) continue;
             const size_t lc = sizeof(T) * 2 * LPN(3 * nl * L);
@@ -530,7 +536,9 @@ struct Engine : EngineBase {
             lds_colp = lc;
             pcol = q;
         }
-        if (!colp) return MRMG_OK;
+        FFTPlan q;
+        if (factorize(vL(), q, col_radix)) pcol = q;
+        else col_radix = 16;
         RCHK(upload_twiddles(pcol, twy));
         lds_rowT = sizeof(T) * 2 * LPN((TYr_eff() / 2) * c->fx);
         CBc = std::max(1, std::min(16, 2048 / pcol.n));
@@ -548,6 +556,29 @@ struct Engine : EngineBase {
             RCHK(tws.upload(t.data(), t.size(), c->stream));
             HIPCHK(hipStreamSynchronize(c->stream));
         }
+        return MRMG_OK;
+    }
+    // the default row threads (init_fft)
+    int row_default() const
+    {
+        const int nx = c->fx;
+        return split ? (nx >= 1024 || (subR > 1 && TYr_eff() * nx >= 4096) ? 256 : 128) : 3 * nx <= 256 ? 128 : 256;
+    }
+    // the layout of the columns for a tensor of z-offset blocks (toeplitz) or layer pairs in
+    // nslot slots, before its spectra are stored; a tensor of the other layout is dropped
+    int fit_split(bool toeplitz)
+    {
+        const bool one = (toeplitz || c->nl == 1) && nslot == 6;   // one layer: one block either way
+        if (fused_ok || sizeof(T) != 8 || c->nl > 4 || one == one_fit) return MRMG_OK;
+        tensor_ok = false;
+        HIPCHK(hipStreamSynchronize(c->stream));
+        const bool def = row_threads == row_def;
+        RCHK(choose_split(one));
+        row_def = row_default();
+        if (def) row_threads = row_def;
+        RCHK(shapes());
+        RCHK(lds_attr());
+        one_fit = one;
         return MRMG_OK;
     }
     // the columns as laid out: vnx() per plane, of vL() values
@@ -707,6 +738,7 @@ struct Engine : EngineBase {
         else if (k == "row_radix") *v = row_radix;
         else if (k == "col_radix") *v = col_radix;
         else if (k == "tensor_offsets") *v = toep ? 1 : 0;
+        else if (k == "col_split") *v = colp ? subR : 0;
         else return set_err(MRMG_ERR_ARG, "unknown tunable '%s'", k.c_str());
         return MRMG_OK;
     }
@@ -1220,7 +1252,7 @@ struct Engine : EngineBase {
         static const int fused[3] = {K_ROW_FWD, K_COL, K_ROW_INV};
         static const int splitc[5] = {K_ROW_FWD, K_COLF, K_PROD, K_COLI, K_ROW_INV};
         static const int prec[4] = {K_ROW_FWD, K_COLF, K_COL, K_ROW_INV};
-        const bool one = split && colp && toep && nslot == 6;
+        const bool one = split && colp;
         const int* seq = one ? fused : split ? splitc : pre ? prec : fused;
         const int n = one ? 3 : split ? 5 : pre ? 4 : 3;
         for (int i = 0; i < n; i++) {

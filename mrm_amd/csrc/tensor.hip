@@ -242,6 +242,7 @@ int Engine<T>::set_tensor_planes(const double* d_real, bool toeplitz)
     // 2 nl - 1 z offsets (block d + nl - 1 for d = ko - ks); planes of the FFT grid
     const int nx = c->fx, ny = c->fy, nxh = c->nxh, nl = c->nl;
     const int nq = toeplitz ? 2 * nl - 1 : nl * nl;
+    RCHK(fit_split(toeplitz));
     const int P = 9 * nq;
     DBuf<C2<double>> TC, tdx, tdy;
     RCHK(TC.alloc((size_t)P * nxh * ny));
