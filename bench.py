@@ -84,7 +84,7 @@ def media_counts(med):
     return cm, runs, E
 
 
-def kernel_bytes(med, P, offsets, fft=None):
+def kernel_bytes(med, P, offsets, fft=None, radix=0):
     """Algorithmic bytes per launch of each kernel class (P: bytes of the demag path's real
     type; the grain state is FP64 in both forms).  Row r2c: the grains' magnetisation
     (3 P per grain), the row-major run lists (geometry and grain, 8 per run, plus the row
@@ -96,7 +96,8 @@ def kernel_bytes(med, P, offsets, fft=None):
     layer reciprocity), or 6 (2 n_lay - 1) when the stored tensor is the z-offset form
     and that is fewer.  With open boundaries (fft = the padded grid) Kc counts the padded
     grid, and the row kernels and the column kernels' media side move only the ny media
-    rows of each column.  A grain stage: ~25 doubles per grain (state, constants, dm,
+    rows of each column; where the row kernels take a radix of the column transform (radix >
+    1) they hand over the padded length.  A grain stage: ~25 doubles per grain (state, constants, dm,
     thermal, field), the exchange CSRs (4 + 8 per entry), the grain's run offsets (4), its
     runs' FP64 field sums, geometry and rows (32 per run) and its magnetisation out to the
     row kernels (3 P)."""
@@ -111,7 +112,8 @@ def kernel_bytes(med, P, offsets, fft=None):
     if offsets:
         tu = min(tu, 6 * (2 * nl - 1))
     half = 6 * nl * kc * P                                 # one pass over the spectra
-    media_rows = 6 * nl * (fx // 2 + 1) * med.ny * P       # the rows the row kernels touch
+    # the values of the spectra that the row kernels touch
+    media_rows = half if radix > 1 else 6 * nl * (fx // 2 + 1) * med.ny * P
     return {
         "row_fwd": 3 * P * G + 8 * runs + rows + media_rows,
         "col": media_rows + media_rows + 2 * tu * kc * P,
@@ -131,7 +133,7 @@ def kernel_table(x, med, P, steps, t0, log, tag, fft=None):
     x.step(steps, t0=t0, philox_seed=SEED, diag=False)
     st = x.kernel_stats()
     x.profile(False)
-    kb = kernel_bytes(med, P, x.get_tune("tensor_offsets"), fft=fft)
+    kb = kernel_bytes(med, P, x.get_tune("tensor_offsets"), fft=fft, radix=x.get_tune("col_split"))
     tot = sum(ms for n, ms in st.values() if n > 0)
     kern = {}
     for k, (n, ms) in st.items():
@@ -166,17 +168,17 @@ def kernel_class(name):
     n = (name[5:] if name.startswith("void ") else name).split("(")[0]
     base = n.split("<")[0].strip()
     args = [s.strip() for s in n[n.find("<") + 1:n.rfind(">")].split(",")] if "<" in n else []
-    if base in ("k_rowT_fwd", "k_row_fwd"):
+    if base in ("k_rowT_fwd", "k_rowS_fwd", "k_row_fwd"):
         return "row_fwd"
-    if base in ("k_rowT_inv", "k_row_inv"):
+    if base in ("k_rowT_inv", "k_rowS_inv", "k_row_inv"):
         return "row_inv"
     if base == "k_colT":
         return "col_inv" if args[2] == "true" else "col_fwd"
     if base in ("k_prod", "k_prod_offsets"):
         return "prod"
-    if base == "k_col":
+    if base in ("k_col", "k_colp"):
         return "col"
-    if base == "k_grain":
+    if base in ("k_grain", "k_grain_batch"):
         return "grain2" if args[1] in ("1", "3") else "grain1"
     if base == "k_copy16":
         return "copy16"
