@@ -1,0 +1,82 @@
+"""The split of the FP64 column transform with radix 2 on open boundaries (one media row a
+group: two items exchange their rows between lanes), with odd column lengths, and under the
+tunables of the row and column kernels: the demag field against the convolution in numpy's
+FFTs (1e-12 of the largest field, as in the split transform's own test), and the launch
+shapes that leave the values unchanged bit for bit.  A captured batch whose column or row
+kernels ask for more than 64 KB of LDS, with a context of another size beside it."""
+import pytest
+
+from mrm_amd import media
+from mrm_amd.llg import Llg, step_batch
+from tests.test_gpu_batch import same, states
+from tests.test_gpu_split_layout import context, convolution_error, load
+
+pytestmark = pytest.mark.gpu
+
+
+# 768, 540 and 810 rows of FFT: radix 4 would leave columns under 256
+@pytest.mark.parametrize("nx,ny,nl", [(32, 384, 3), (30, 270, 4), (20, 405, 3), (64, 384, 4)])
+@pytest.mark.parametrize("tune", [{}, {"row_block": 2}, {"row_block": 4, "row_threads": 64},
+                                  {"row_threads": 256, "col_radix": 4}, {"row_radix": 4, "col_radix": 8}])
+def test_radix_two_open(nx, ny, nl, tune):
+    x, med = context(nx, ny, nl, 2e-7, True)
+    N = x.build_tensor(num_images=0, return_real=True)
+    load(x, med)
+    for k, v in tune.items():
+        x.tune(k, v)
+    x.step(0, diag=False)
+    assert x.get_tune("col_split") == 2
+    for k, v in tune.items():
+        assert x.get_tune(k) == v
+    assert convolution_error(x, med, N) <= 1e-12
+    x.close()
+
+
+@pytest.mark.parametrize("nx,ny,nl,open_,radix", [
+    (32, 384, 3, True, 2), (20, 405, 3, True, 2), (30, 540, 2, True, 4), (32, 1024, 3, True, 8), (45, 540, 4, False, 2),
+    (32, 1024, 4, False, 4), (40, 2048, 4, False, 8)])
+def test_row_shapes_leave_the_values(nx, ny, nl, open_, radix):
+    def run(tune):
+        med = media.make_media(nx, ny, dz=2e-7, n_lay=nl, seed=3, thermal=True, temperature=300.0)
+        x = Llg(nx, ny, nl, med.dx, med.dy, med.dz, open=open_)
+        x.build_tensor(num_images=0)
+        x.set_media(med)
+        x.set_llg(dt=5e-14)
+        for k, v in tune.items():
+            x.tune(k, v)
+        assert x.get_tune("col_split") == radix
+        x.step(3, philox_seed=7)
+        out = states(x, nl)
+        x.close()
+        return out
+
+    want = run({})
+    for tune in ({"row_block": 2}, {"row_block": 4}, {"row_threads": 64}, {"row_threads": 256}, {"wave_fft": 1}):
+        assert same(want, run(tune))
+
+
+@pytest.mark.parametrize("nx,ny,nl", [(24, 4096, 4), (1024, 2304, 1)])   # 98 KB a column kernel; 70 KB a row kernel
+def test_captured_batch_with_wide_lds(nx, ny, nl):
+    med = media.make_media(nx, ny, dz=2e-7, n_lay=nl, seed=3, thermal=True, temperature=300.0)
+
+    def member():
+        x = Llg(nx, ny, nl, med.dx, med.dy, med.dz)
+        x.build_tensor(num_images=0)
+        x.set_media(med)
+        x.set_llg(dt=5e-14)
+        return x
+
+    solo, batch = [member() for _ in range(2)], [member() for _ in range(2)]
+    assert solo[0].get_tune("col_split") > 1
+    other, m2 = context(24, 3072, 4, 2e-7)      # 74 KB a column kernel
+    other.build_tensor(num_images=0)
+    load(other, m2)
+    other.step(1)
+    for x, p in zip(solo, (7, 8)):
+        x.step(4, philox_seed=p)
+    t = step_batch(batch, 2, philox_seeds=[7, 8], graph=True)
+    other.step(1)
+    step_batch(batch, 2, philox_seeds=[7, 8], t0s=t, graph=True)
+    assert all(same(states(a, nl), states(b, nl)) for a, b in zip(solo, batch))
+    for x in solo + batch + [other]:
+        x.close()
