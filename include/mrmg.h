@@ -388,7 +388,10 @@ int mrmg_profile(mrmg_ctx *ctx, int enable);
  * "lanes_per_grain" (1, 2, 4, 8, 16).  The thread counts, "col_groups", "row_block" and
  * (with "wave_fft" 0) "col_path" leave results unchanged bit for bit; the others may
  * change the order of floating-point operations (FFT factorisation, gather sums) and so
- * the last bits.  A combination that does not fit the grid is refused. */
+ * the last bits.  A combination that does not fit the grid is refused.  "col_threads" is
+ * 512 or 1024 by the grid, the tensor and the other shapes unless another value is set; a
+ * value equal to that choice leaves it to them, so that mrmg_get_tune's can be written back
+ * without effect.  (A batch runs with 512 where the choice is 1024.) */
 int mrmg_tune(mrmg_ctx *ctx, const char *key, int value);
 /* The value of a tunable, or of the read-only key "tensor_offsets": 1 when the stored
  * tensor spectra are the 2 n_lay - 1 z-offset blocks (the tensor depends on the layer pair

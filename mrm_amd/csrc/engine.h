@@ -318,10 +318,11 @@ struct Engine : EngineBase {
     bool cells_out = false;
     DBuf<int> slot2c;
     // launch shapes (mrmg_tune): threads of the row and column workgroups, observation-layer
-    // groups per column workgroup, lanes per grain in the grain kernels
+    // groups per column workgroup, lanes per grain in the grain kernels.  col_threads: unless
+    // col_rule decides (col_set)
     int row_threads = 128, col_threads = 512, kg = 1, lpg = 8;
     int row_def = 128;      // the row threads that were not asked for (row_th)
-    bool col_set = false;   // col_threads was asked for
+    bool col_set = false;   // col_threads is other than col_rule's
     int maxb_big = -1;      // elements per lane of the column kernel at 1024 threads
     bool lpg_set = false;   // lanes_per_grain was tuned: build() leaves it
     // split column path (column-contiguous spectra): rows per row workgroup, columns per
@@ -663,9 +664,12 @@ struct Engine : EngineBase {
             if (v != 256 && v != 512 && v != 1024) return set_err(MRMG_ERR_ARG, "col_threads must be 256, 512 or 1024");
             if (v > 512 && nslot != 6)
                 return set_err(MRMG_ERR_UNSUPPORTED, "col_threads 1024 needs the symmetric (6-slot) tensor");
-            old = col_threads; col_threads = v;
-            if (shapes() != MRMG_OK) { col_threads = old; return shapes(), MRMG_ERR_UNSUPPORTED; }
-            col_set = true;
+            // what the rule takes by itself stays its own, so that a value read and written back
+            // changes nothing
+            const bool os = col_set;
+            col_set = v != col_rule();
+            old = col_threads; col_threads = col_set ? v : 512;
+            if (shapes() != MRMG_OK) { col_threads = old; col_set = os; return shapes(), MRMG_ERR_UNSUPPORTED; }
         } else if (k == "col_groups") {
             if (v < 1 || v > c->nl) return set_err(MRMG_ERR_ARG, "col_groups must be in 1..n_lay");
             old = kg; kg = v;
@@ -729,7 +733,7 @@ struct Engine : EngineBase {
     {
         std::string k(key ? key : "");
         if (k == "row_threads") *v = row_threads;
-        else if (k == "col_threads") *v = col_threads;
+        else if (k == "col_threads") *v = col_th();
         else if (k == "col_groups") *v = kg;
         else if (k == "lanes_per_grain") *v = lpg;
         else if (k == "col_path") *v = split ? 1 : pre ? 3 : tl ? 2 : 0;
@@ -745,7 +749,7 @@ struct Engine : EngineBase {
 
     // Threads of the fused path's row workgroups.  A batch can have more of them than the chip
     // holds at once with 256 threads (FP32 seven a CU, FP64 five, by their registers).  Then
-    // rows of up to 300 points take 128, unless the threads were asked for: a step of batches
+    // rows of up to 300 points take 128, unless other threads were asked for: a step of batches
     // with 128 / 256, us, FP32 128x128x2 1024 workgroups 92 / 91, 1536 124 / 125, 2048
     // 134 / 150, 4096 212 / 233; 288x128x2 1536 196 / 188, 2048 230 / 238; FP64 128x128x2 1024
     // 115 / 114, 1536 137 / 153; 288x128x2 1024 188 / 176, 1536 233 / 241.  From 320 points on a
@@ -764,11 +768,12 @@ struct Engine : EngineBase {
     // at 450x405x3 FP32, but 33 against 24 at 512x512x2 (257 workgroups) and 18.6 against 13.4
     // at 512x256x1 (one item a thread of 256).
     // Only where the 1024-thread kernel is built: one context, 6 slots, no wave-local FFTs.
-    int col_th() const
+    int col_th() const { return col_set ? col_threads : col_rule(); }
+    int col_rule() const
     {
         const int per = (c->nl + kg - 1) / kg;
         const bool fits = !btab && !wv && !pre && nslot == 6 && maxb_big > 0 && maxb_big <= 16 && per * c->fy <= 2048;
-        return !col_set && fits && per * c->fy > 512 && c->nxh * kg <= 256 ? 1024 : col_threads;
+        return fits && per * c->fy > 512 && c->nxh * kg <= 256 ? 1024 : 512;
     }
     template <int MB> int lds_attr_mb();
     template <int MB> int lds_attr_col();
