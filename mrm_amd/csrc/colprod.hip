@@ -85,15 +85,22 @@ __global__ void __launch_bounds__(512) k_colp(DemagOps<T> one, const DemagOps<T>
     }
 }
 
-template <typename T, int E, int NL>
-static int launch_colp_nl(hipStream_t s, int z, int threads, size_t lds, const DemagOps<T>& o, const DemagOps<T>* tab,
-                          int L, int vnx, const FFTPlan& py, const C2<T>* twy)
+// the kernel's dynamic LDS at most (choose_split): with 512 threads 14 elements a thread, with
+// 256 for up to 56 KB as well
+#define MRMG_COLP_LDS (112 * 1024)
+#define MRMG_COLP_E 16
+
+#define COLP_FN(NL) ((const void*)k_colp<double, MRMG_COLP_E, NL>)
+#define COLP_NL(M) M(1) M(2) M(3) M(4)
+
+// dynamic LDS above 64 KiB must be requested: the most that any context's kernel takes, so that
+// one context's request is not another's limit
+template <>
+int Engine<double>::lds_attr_colp()
 {
-    if (lds > 64 * 1024)   // dynamic LDS above 64 KiB must be requested
-        HIPCHK(hipFuncSetAttribute((const void*)k_colp<T, E, NL>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL((k_colp<T, E, NL>), dim3((unsigned)((vnx + 7) / 8 * 8), 1, (unsigned)z), dim3(threads), lds, s, o,
-                       tab, L, vnx, py, twy);
-    HIPCHK(hipGetLastError());
+#define COLP_ATTR(NL) HIPCHK(hipFuncSetAttribute(COLP_FN(NL), hipFuncAttributeMaxDynamicSharedMemorySize, MRMG_COLP_LDS));
+    COLP_NL(COLP_ATTR)
+#undef COLP_ATTR
     return MRMG_OK;
 }
 
@@ -101,15 +108,21 @@ template <>
 int Engine<double>::launch_colp()
 {
     const DemagOps<double> o = ops();
-    const int z = btab ? bn : 1, L = vL(), th = colp_threads, e = pick_e(3 * c->nl, pcol, th);
-    if (e < 0 || e > 32 || nslot != 6 || !one_fit) return set_err(MRMG_ERR_STATE, "the one-kernel column path does not fit");
-#define KCN(N)                                                                                                          \
-    case N:                                                                                                             \
-        return e > 16 ? launch_colp_nl<double, 32, N>(c->stream, z, th, lds_colp, o, btab, L, vnx(), pcol, twy.p)       \
-                      : launch_colp_nl<double, 16, N>(c->stream, z, th, lds_colp, o, btab, L, vnx(), pcol, twy.p);
+    const int z = btab ? bn : 1, L = vL(), vx = vnx(), th = colp_threads, e = pick_e(3 * c->nl, pcol, th);
+    if (e < 0 || e > MRMG_COLP_E || lds_colp > MRMG_COLP_LDS || nslot != 6 || !one_fit)
+        return set_err(MRMG_ERR_STATE, "the one-kernel column path does not fit");
+    const dim3 g((unsigned)((vx + 7) / 8 * 8), 1, (unsigned)z);
+#define COLP_LAUNCH(NL)                                                                                                 \
+    case NL:                                                                                                            \
+        hipLaunchKernelGGL((k_colp<double, MRMG_COLP_E, NL>), g, dim3(th), lds_colp, c->stream, o, btab, L, vx, pcol,   \
+                           twy.p);                                                                                      \
+        break;
     switch (c->nl) {
-        KCN(1) KCN(2) KCN(3) KCN(4)
+        COLP_NL(COLP_LAUNCH)
+    default:
+        return set_err(MRMG_ERR_STATE, "the one-kernel column path is not built for %d layers", c->nl);
     }
-#undef KCN
-    return set_err(MRMG_ERR_STATE, "the one-kernel column path is not built for %d layers", c->nl);
+#undef COLP_LAUNCH
+    HIPCHK(hipGetLastError());
+    return MRMG_OK;
 }

@@ -590,6 +590,10 @@ int Engine<T>::lds_attr()
         RCHK(lds_attr_split<4>()); RCHK(lds_attr_split<8>()); RCHK(lds_attr_split<16>());
         RCHK(lds_attr_split<32>()); RCHK(lds_attr_split<64>());
     }
+    if constexpr (sizeof(T) == 8) {
+        if (colp && lds_colp > 64 * 1024) RCHK(lds_attr_colp());
+        if (subR > 1 && lds_rowT > 64 * 1024) RCHK(lds_attr_rowS());
+    }
     return MRMG_OK;
 }
 

@@ -529,7 +529,7 @@ struct Engine : EngineBase {
             const size_t lc = sizeof(T) * 2 * LPN(3 * nl * L);
             const int th = lc > 56 * 1024 ? 512 : 256, e = pick_e(3 * nl, q, th);
             if (lc > 112 * 1024 || ty / 2 * c->fx > 4096 || ty > 16) continue;
-            if (pick_e(ty / 2, c->px, 256) < 0 || e < 0 || e > 32) continue;
+            if (pick_e(ty / 2, c->px, 256) < 0 || e < 0) continue;   // e: 14 at most, of 16
             subR = R;
             subRm = rm;
             colp = true;
@@ -1317,6 +1317,8 @@ struct Engine : EngineBase {
         return (unsigned)(((n + per - 1) / per * 3 * c->nl + 7) / 8 * 8);
     }
     int launch_colp();
+    int lds_attr_colp();
+    int lds_attr_rowS();
     int launch_rowS(bool inv, dim3 g, dim3 b);   // the split transform's row kernels (rowsplit.hip)
     template <int MB> void launch_rowT_fwd(dim3 g, dim3 b);
     template <int MB> void launch_colT_fwd(dim3 g, dim3 b);

@@ -308,12 +308,6 @@ static int rowS(bool inv, bool cells, dim3 g, dim3 b, size_t lds, hipStream_t s,
                 const DemagOps<double>* tab, const mrmg_ctx* c, int TY, const FFTPlan& px, const C2<double>* tw,
                 const RowSplit<double>& rs)
 {
-    const hipFuncAttribute a = hipFuncAttributeMaxDynamicSharedMemorySize;   // above 64 KiB it must be requested
-    if (lds > 64 * 1024) {
-        HIPCHK(hipFuncSetAttribute((const void*)k_rowS_fwd<double, E>, a, (int)lds));
-        HIPCHK(hipFuncSetAttribute((const void*)k_rowS_inv<double, E, false>, a, (int)lds));
-        HIPCHK(hipFuncSetAttribute((const void*)k_rowS_inv<double, E, true>, a, (int)lds));
-    }
     if (!inv)
         hipLaunchKernelGGL((k_rowS_fwd<double, E>), g, b, lds, s, o, tab, c->fx, c->ny, c->fy, c->nl, c->nxh, TY, px, tw,
                            rs);
@@ -324,6 +318,25 @@ static int rowS(bool inv, bool cells, dim3 g, dim3 b, size_t lds, hipStream_t s,
         hipLaunchKernelGGL((k_rowS_inv<double, E, false>), g, b, lds, s, o, tab, c->fx, c->ny, c->fy, c->nx, c->nl,
                            c->nxh, TY, px, tw, rs);
     HIPCHK(hipGetLastError());
+    return MRMG_OK;
+}
+
+// as lds_attr_colp; SplitRuns takes 132 bytes of the 160 KB
+template <int E>
+static int rowS_attr()
+{
+    const hipFuncAttribute a = hipFuncAttributeMaxDynamicSharedMemorySize;
+    const int lds = 160 * 1024 - 256;
+    HIPCHK(hipFuncSetAttribute((const void*)k_rowS_fwd<double, E>, a, lds));
+    HIPCHK(hipFuncSetAttribute((const void*)k_rowS_inv<double, E, false>, a, lds));
+    HIPCHK(hipFuncSetAttribute((const void*)k_rowS_inv<double, E, true>, a, lds));
+    return MRMG_OK;
+}
+
+template <>
+int Engine<double>::lds_attr_rowS()
+{
+    RCHK(rowS_attr<4>()); RCHK(rowS_attr<8>()); RCHK(rowS_attr<16>()); RCHK(rowS_attr<32>()); RCHK(rowS_attr<64>());
     return MRMG_OK;
 }
 
