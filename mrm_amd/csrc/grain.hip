@@ -1020,7 +1020,8 @@ __device__ __forceinline__ void grain_body(const GrainData<T>& gd, T* __restrict
     T h[3] = {0, 0, 0};
     double tev[2] = {0, 0};   // grain temperature now and at the next evaluation (moving sources)
     GrainSums S;
-    if (ngw > 0 && (MODE != GM_PUSH1 || gd.n_temp > 0)) {
+    // (the push from stored fields takes this evaluation's temperature from tlast)
+    if (ngw > 0 && (MODE != GM_PUSH1 || gd.n_temp > 1)) {
         if constexpr (WAVE)
             grain_sums<T, LPG>(gd, slp, gw0, ngw, mf, Hr, MODE == GM_PUSH1,
                                gval + wv * GrainShape<LPG>::doubles(gd.n_temp), S);
@@ -1034,11 +1035,7 @@ __device__ __forceinline__ void grain_body(const GrainData<T>& gd, T* __restrict
     } else {
 #pragma unroll
         for (int c = 0; c < 3; c++) h[c] = hout[(size_t)c * G + g];
-        if (tsrc) {
-            const double dc = (double)P.cells;
-            tev[0] = S.t[0] / dc + g_temp;
-            if (gd.n_temp > 1) tev[1] = S.t[1] / dc + g_temp;
-        }
+        if (tsrc && gd.n_temp > 1) tev[1] = S.t[1] / (double)P.cells + g_temp;
     }
     T mo[3] = {0, 0, 0};
     T fsc = 0;   // Ms * ms_scale of the new state: the cell magnetisation factor
