@@ -391,7 +391,11 @@ int mrmg_profile(mrmg_ctx *ctx, int enable);
  * the last bits.  A combination that does not fit the grid is refused.  "col_threads" is
  * 512 or 1024 by the grid, the tensor and the other shapes unless another value is set; a
  * value equal to that choice leaves it to them, so that mrmg_get_tune's can be written back
- * without effect.  (A batch runs with 512 where the choice is 1024.) */
+ * without effect.  (A batch runs with 512 where the choice is 1024.)  Row kernels that
+ * take a radix of the column transform ("col_split" below, 2 and more) hold whole groups of
+ * that many rows (half as many with open boundaries): a smaller "row_block" is raised to
+ * them, and mrmg_get_tune says to what.  They have no wave-local form: "wave_fft" is kept
+ * for a tensor of another kind and has no effect meanwhile. */
 int mrmg_tune(mrmg_ctx *ctx, const char *key, int value);
 /* The value of a tunable, or of the read-only key "tensor_offsets": 1 when the stored
  * tensor spectra are the 2 n_lay - 1 z-offset blocks (the tensor depends on the layer pair

@@ -737,7 +737,7 @@ struct Engine : EngineBase {
         else if (k == "col_groups") *v = kg;
         else if (k == "lanes_per_grain") *v = lpg;
         else if (k == "col_path") *v = split ? 1 : pre ? 3 : tl ? 2 : 0;
-        else if (k == "row_block") *v = TYr;
+        else if (k == "row_block") *v = TYr_eff();
         else if (k == "wave_fft") *v = wv ? 1 : 0;
         else if (k == "row_radix") *v = row_radix;
         else if (k == "col_radix") *v = col_radix;

@@ -80,3 +80,16 @@ def test_captured_batch_with_wide_lds(nx, ny, nl):
     assert all(same(states(a, nl), states(b, nl)) for a, b in zip(solo, batch))
     for x in solo + batch + [other]:
         x.close()
+
+
+@pytest.mark.parametrize("nx,ny,nl,open_,rows", [(40, 2048, 4, False, 8), (32, 1024, 4, False, 4), (32, 1024, 3, True, 4),
+                                                 (32, 384, 3, True, 1)])
+def test_row_block_reads_what_is_launched(nx, ny, nl, open_, rows):
+    x, med = context(nx, ny, nl, 2e-7, open_)
+    x.build_tensor(num_images=0)
+    for v in (2, 4, 8):
+        x.tune("row_block", v)
+        assert x.get_tune("row_block") == max(v, rows)
+        x.tune("row_block", x.get_tune("row_block"))
+        assert x.get_tune("row_block") == max(v, rows)
+    x.close()
