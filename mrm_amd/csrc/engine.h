@@ -677,9 +677,9 @@ struct Engine : EngineBase {
         } else if (k == "lanes_per_grain") {
             if (v != 1 && v != 2 && v != 4 && v != 8 && v != 16)
                 return set_err(MRMG_ERR_ARG, "lanes_per_grain must be 1, 2, 4, 8 or 16");
+            if (nruns > 0) RCHK(order_sums(v));
             lpg = v;
             lpg_set = true;
-            if (nruns > 0) RCHK(order_sums());
         } else if (k == "col_path") {
             if (v < 0 || v > 3)
                 return set_err(MRMG_ERR_ARG, "col_path must be 0 (fused), 1 (split), 2 (fused, column-contiguous) or 3 "
@@ -1010,11 +1010,11 @@ struct Engine : EngineBase {
     // 22 884).  A wave that stages 64 grains' runs has the index loads in flight together, and
     // there the row kernels' consecutive stores count.
     static bool sums_by_grain(int lanes) { return lanes > 1; }
-    // the map for the current lanes: its inverse, where the order changes (the sums themselves
-    // are rewritten before they are read)
-    int order_sums()
+    // the map for these lanes: its inverse, where the order changes (the sums themselves are
+    // rewritten before they are read)
+    int order_sums(int lanes)
     {
-        if (sums_by_grain(lpg) == by_grain) return MRMG_OK;
+        if (sums_by_grain(lanes) == by_grain) return MRMG_OK;
         std::vector<int> a(nruns), b(nruns);
         HIPCHK(hipMemcpyAsync(a.data(), run_map.p, sizeof(int) * nruns, hipMemcpyDeviceToHost, c->stream));
         HIPCHK(hipStreamSynchronize(c->stream));

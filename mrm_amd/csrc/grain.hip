@@ -319,13 +319,14 @@ __device__ __forceinline__ void grain_sums(const GrainData<T>& gd, const LayerPa
 template <int LPG, int U> struct LaneRound {
     int q[U], nb[U], geo[U], row[U];
     double w[U];
+    // src: the runs' places too; the run sums are in the grain's own order (sums_by_grain)
     template <typename T>
     __device__ __forceinline__ void load(const GrainData<T>& gd, int r0, int r1, int x0, int x1, int b, bool src)
     {
 #pragma unroll
         for (int u = 0; u < U; u++) {
             const int r = r0 + b + u * LPG, e = x0 + b + u * LPG, rc = r < r1 ? r : r0, ec = e < x1 ? e : x0;
-            q[u] = gd.run_q ? at32(gd.run_q, rc) : rc;
+            q[u] = rc;
             nb[u] = at32(gd.x_nb, ec);
             w[u] = at32(gd.x_w, ec);
             if (src) {
@@ -343,14 +344,14 @@ template <int LPG, int U> struct LaneRound {
 // loads and nothing else, so a layer without a source has a loop of its own, of two runs and
 // entries a lane and round: as one loop with the sources' branches, a round of one entry a
 // lane and 8 lanes, a second round was due for every ninth neighbour and a stage took 0.2 us
-// more (64x64x1: 8.65 now), and two stages with 4 lanes took 23.2 against 21.2 us (31 302
+// more (64x64x1), and two stages with 4 lanes took 23.2 against 21.2 us (31 302
 // grains) and 59 against 48 (119 640).
-template <typename T, int LPG>
+template <typename T, int LPG, bool SRC>
 __device__ __forceinline__ void grain_sums_lanes(const GrainData<T>& gd, const LayerParams* lp, int k, int fk, int tk,
                                                  int lane, int r0, int r1, int x0, int x1, const T* __restrict__ mf,
                                                  const double* __restrict__ Hr, bool temps_only, GrainSums& S)
 {
-    const int G = gd.G, nt = gd.n_temp;
+    const int G = gd.G, nt = SRC ? gd.n_temp : 0;
     const bool fsrc = !temps_only && fk == MRMG_SRC_FIELD_TABLE;
     const bool tsrc = nt > 0 && tk != MRMG_SRC_NONE, tsg = tsrc && tk == MRMG_SRC_TEMP_SG;
     const size_t NR = (size_t)gd.nruns;
@@ -386,7 +387,7 @@ __device__ __forceinline__ void grain_sums_lanes(const GrainData<T>& gd, const L
                 }
             }
         }
-    } else {
+    } else if constexpr (SRC) {
         constexpr int U = LPG <= 4 ? 2 : 1;
         for (int b = lane; b < n; b += U * LPG) {
             LaneRound<LPG, U> I;
@@ -938,7 +939,11 @@ __device__ __forceinline__ void rot_push(int type, T scale1, T scale2, const T* 
 }
 
 
-template <typename T, int MODE, int LPG, typename TC>
+// SRC: some layer has a moving source.  Without one, a kernel of several lanes a grain has none
+// of the sources' code: their tables' addresses took more scalar registers than there are, so
+// that the arguments were loaded, waited for and put aside in several rounds (64x64x1 FP64 a
+// stage 8.8 us with it, 8.2 without; 128x128x4 9.0 and 8.2; 187 vector registers, 138).
+template <typename T, int MODE, int LPG, typename TC, bool SRC>
 __device__ __forceinline__ void grain_body(const GrainData<T>& gd, T* __restrict__ ma, T* __restrict__ mb,
                                            T* __restrict__ dm, T* __restrict__ hthm, T* __restrict__ hout,
                                            const double* __restrict__ Hr, TC* __restrict__ Mg, const StepArgs& a,
@@ -1015,18 +1020,19 @@ __device__ __forceinline__ void grain_body(const GrainData<T>& gd, T* __restrict
         for (int i = threadIdx.x; i < DIAG_STRIDE; i += 256) red[i] = 0.0;
     __syncthreads();
     const LayerParams& L = slp[k];
-    const int fk = L.src[0].kind, tk = L.src[1].kind;   // read once: each LDS read is waited for in turn
+    // read once: each LDS read is waited for in turn
+    const int fk = SRC ? L.src[0].kind : MRMG_SRC_NONE, tk = SRC ? L.src[1].kind : MRMG_SRC_NONE;
     const bool fsrc = fk == MRMG_SRC_FIELD_TABLE, tsrc = tk != MRMG_SRC_NONE;
     T h[3] = {0, 0, 0};
     double tev[2] = {0, 0};   // grain temperature now and at the next evaluation (moving sources)
     GrainSums S;
     // (the push from stored fields takes this evaluation's temperature from tlast)
-    if (ngw > 0 && (MODE != GM_PUSH1 || gd.n_temp > 1)) {
+    if (ngw > 0 && (MODE != GM_PUSH1 || (SRC && gd.n_temp > 1))) {
         if constexpr (WAVE)
             grain_sums<T, LPG>(gd, slp, gw0, ngw, mf, Hr, MODE == GM_PUSH1,
                                gval + wv * GrainShape<LPG>::doubles(gd.n_temp), S);
         else
-            grain_sums_lanes<T, LPG>(gd, slp, k, fk, tk, ln % LPG, r0, r1, x0, x1, mf, Hr, MODE == GM_PUSH1, S);
+            grain_sums_lanes<T, LPG, SRC>(gd, slp, k, fk, tk, ln % LPG, r0, r1, x0, x1, mf, Hr, MODE == GM_PUSH1, S);
     }
     if (act) {
     if constexpr (LPG < 8) load();
@@ -1209,26 +1215,27 @@ __device__ __forceinline__ void grain_body(const GrainData<T>& gd, T* __restrict
     }
 }
 
-template <typename T, int MODE, int LPG, typename TC>
+template <typename T, int MODE, int LPG, typename TC, bool SRC>
 __global__ void __launch_bounds__(256) k_grain(GrainData<T> gd, T* __restrict__ ma, T* __restrict__ mb,
                                                T* __restrict__ dm, T* __restrict__ hthm, T* __restrict__ hout,
                                                const double* __restrict__ Hr, TC* __restrict__ Mg,
                                                StepArgs a, double* __restrict__ diag_part, T* __restrict__ mc)
 {
-    grain_body<T, MODE, LPG, TC>(gd, ma, mb, dm, hthm, hout, Hr, Mg, a, diag_part, mc);
+    grain_body<T, MODE, LPG, TC, SRC>(gd, ma, mb, dm, hthm, hout, Hr, Mg, a, diag_part, mc);
 }
 
 // One stage of every member of a batch (blockIdx.y the member): a member of some thousand
 // grains fills a small part of the chip, and sixteen launches of it one after the other cost
 // sixteen latencies (16 contexts of 256x256x2, 7 846 grains each: 64 / 53 us a stage against
 // 117 / 101).  a: the stage's times and the push, equal for all; seed and clock are the member's.
+// No member has a moving source.
 template <typename T, int MODE, int LPG, typename TC>
 __global__ void __launch_bounds__(256) k_grain_batch(const GrainOps<T, TC>* __restrict__ tab, StepArgs a)
 {
     const GrainOps<T, TC>& o = tab[blockIdx.y];
     a.seed = o.seed;
     a.clk = o.clk;
-    grain_body<T, MODE, LPG, TC>(o.gd, o.ma, o.mb, o.dm, o.hthm, o.h, o.Hr, o.Mg, a, nullptr, nullptr);
+    grain_body<T, MODE, LPG, TC, LPG == 1>(o.gd, o.ma, o.mb, o.dm, o.hthm, o.h, o.Hr, o.Mg, a, nullptr, nullptr);
 }
 
 // llg()'s loop-top statistics (llg.f90:217-237) of layer blockIdx.x: the volume-weighted
@@ -1476,10 +1483,13 @@ template <int MODE, int LPG> int Engine<T>::launch_grain(const StepArgs& a, S* m
 {
     const size_t threads = (size_t)G * LPG;
     const unsigned nb8 = (unsigned)(((threads + 255) / 256 + 7) / 8 * 8);
-    hipLaunchKernelGGL((k_grain<S, MODE, LPG, T>), dim3(nb8), dim3(256),
-                       LPG == 1 ? 4 * sizeof(double) * GrainShape<LPG>::doubles(n_temp) : 0, c->stream,
-                       gdata(), ma.p, mb.p, dm.p, hthm.p, h.p, demag_on() ? Hr.p : nullptr,
-                       demag_on() ? Mg.p : nullptr, a, diag_part.p, mout);
+    const size_t lds = LPG == 1 ? 4 * sizeof(double) * GrainShape<LPG>::doubles(n_temp) : 0;
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(nb8), dim3(256), lds, c->stream, gdata(), ma.p, mb.p, dm.p, hthm.p, h.p,
+                           demag_on() ? Hr.p : nullptr, demag_on() ? Mg.p : nullptr, a, diag_part.p, mout);
+    };
+    if (LPG == 1 || any_src) launch(k_grain<S, MODE, LPG, T, true>);
+    else launch(k_grain<S, MODE, LPG, T, LPG == 1>);
     HIPCHK(hipGetLastError());
     return MRMG_OK;
 }
