@@ -91,17 +91,23 @@ __device__ __forceinline__ void runs_to_lds(const RowRuns& R, const T* __restric
 }
 
 // The run descriptors a thread sums in lds_to_runs, its first RU of them loaded ahead
-// (at kernel start, before the spectra and the FFT) by prefetch.
-template <int RU>
+// (at kernel start, before the spectra and the FFT) by prefetch.  TO: with the places of the
+// sums, which a short launch would wait for at its end (64x64x4 FP32 c2r 9.3 us without, 9.1
+// with).  Longer rows, of more than 4 FFT elements a thread, do not hold their registers (4 to
+// 8) across the FFT.
+template <int RU, bool TO>
 struct RunsAhead {
     int q0, q1;
-    int geo[RU];
+    int geo[RU], to[TO ? RU : 1];
     __device__ __forceinline__ void fetch(const RowRuns& R, int qb, int nt)
     {
 #pragma unroll
         for (int u = 0; u < RU; u++) {
             const int q = qb + u * nt;
-            if (q < q1) geo[u] = R.geo[q];
+            if (q < q1) {
+                geo[u] = R.geo[q];
+                if constexpr (TO) to[u] = R.perm ? R.perm[q] : q;
+            }
         }
     }
     __device__ __forceinline__ void prefetch(const RowRuns& R, int k, int ny, int y0, int nrows)
@@ -115,17 +121,20 @@ struct RunsAhead {
 
 // The cell field of the same rows, summed over each run (in x order, in FP64) into
 // Hr[c] (c = c0+ci), with the layout of runs_to_lds.
-template <typename T, int NC, int RU>
-__device__ __forceinline__ void lds_to_runs(const RowRuns& R, RunsAhead<RU>& A, double* __restrict__ Hr, int c0,
+template <typename T, int NC, int RU, bool TO>
+__device__ __forceinline__ void lds_to_runs(const RowRuns& R, RunsAhead<RU, TO>& A, double* __restrict__ Hr, int c0,
                                             int nrows, int np, int nx, const T* re, const T* im, const int* roff)
 {
     const int nt = (int)blockDim.x, tid = (int)threadIdx.x;
     int yy = 0;   // increasing q: the row index only moves forward
     for (int qb = A.q0 + tid; qb < A.q1; qb += RU * nt) {
         if (qb != A.q0 + tid) A.fetch(R, qb, nt);
-        int to[RU];   // where the sums go: loaded here, not held across the FFT (4 to 8 registers)
+        int to[RU];
 #pragma unroll
-        for (int u = 0; u < RU; u++) to[u] = R.perm && qb + u * nt < A.q1 ? R.perm[qb + u * nt] : qb + u * nt;
+        for (int u = 0; u < RU; u++) {
+            if constexpr (TO) to[u] = A.to[u];
+            else to[u] = R.perm && qb + u * nt < A.q1 ? R.perm[qb + u * nt] : qb + u * nt;
+        }
 #pragma unroll
         for (int u = 0; u < RU; u++) {
             const int q = qb + u * nt;
@@ -213,7 +222,7 @@ __global__ void __launch_bounds__(256) k_row_inv(DemagOps<T> one, const DemagOps
     T* im = re + LPN(3 * nx);
     const int y0 = 2 * blockIdx.x, y1 = y0 + 1, k = blockIdx.y;
     const bool has1 = y1 < ny;
-    RunsAhead<MRMG_RU(3, E)> ra;
+    RunsAhead<MRMG_RU(3, E), E <= 4> ra;
     if (!CELLS) ra.prefetch(R, k, ny, y0, has1 ? 2 : 1);
     staged_load<(E < 4 ? E : 4)>(
         3 * nxh,
@@ -496,7 +505,7 @@ __global__ void __launch_bounds__(256) k_rowT_inv(DemagOps<T> one, const DemagOp
     const int k = kc / 3, c = kc - 3 * k;
     const C2<T>* src = S + (size_t)kc * nxh * sy;
     const int nrows = min(TY, ny - y0);
-    RunsAhead<MRMG_RU(1, E)> ra;
+    RunsAhead<MRMG_RU(1, E), false> ra;
     if (!CELLS) ra.prefetch(R, k, ny, y0, nrows);
     // each thread takes one (kx, row pair) and forms z = A + iB at kx and its mirror.  B =
     // TY/2 is 1, 2 or 4: kx and p are a shift and a mask of idx
