@@ -502,16 +502,27 @@ struct Engine : EngineBase {
 
     // The split of the column transform over the row kernels (RowSplit), for which the columns
     // left between them go through one kernel (forward transform, product and inverse in LDS,
-    // colprod.hip) instead of three passes over memory.  FP64 only: in FP32 the other order of
-    // the transform's steps moves a run's mean magnetisation by more than 1e-9.  Taken with the
-    // largest radix for which
-    // * a column keeps 256 values, one a thread of the product (FP32, columns of 1024 values
-    //   of 8 layers: radix 4 takes 138 us a field for the columns, radix 8 190);
-    // * 3 n_lay columns are at most 112 KB (512x4096x4: radix 8 of 98 KB, one workgroup a CU,
-    //   271 us a field against 380 in three kernels; rows 122 / 126 against 102 / 105);
-    // * the product's registers hold the layers (4);
+    // colprod.hip) instead of three passes over memory.  FP64 only: FP32 keeps the order of the
+    // transform's steps, and with it its roundings.  Taken with the largest radix for which
+    // (figures: a field's demag kernels in us, three column kernels / one)
+    // * a column keeps 256 values, one a thread of the product;
+    // * 3 n_lay columns are at most 112 KB (512x4096x4, radix 8 of 98 KB: 588 / 540);
+    // * the product's registers hold the layers (4).  With four they leave eight waves a CU, and
+    //   three workgroups of 256 values or one of 360 to 512 fill it best: 256 values (radix 4)
+    //   512x1024x4 181 / 125, open 256x512x4 140 / 100; 360 to 500 (radix 2) 512x720x4
+    //   157 / 151, 800 172 / 147, 900 183 / 184, 1000 190 / 176; but 270 to 320 64x540x4 57 / 60,
+    //   512x600x4 123 / 130, 2048x640x4 367 / 385, 512x2160x4 364 / 370, 540 (radix 4) 364 / 375.
+    //   Open columns move their padding in one kernel and not in three: 256x300x4 110 / 120, 405
+    //   140 / 154, 500 148 / 154; of three layers with radix 8 512x1080x3 385 / 427, but 256 values
+    //   512x1024x3 314 / 294, and with less 256x405x3 120 / 102, 256x540x3 133 / 122;
     // * the row kernels' rows take at most 4096 transform elements (70 KB; 64 a thread with
-    //   the fewest threads that can be asked for).
+    //   the fewest threads that can be asked for): 2048x2160x1, radix 4, 323 / 303, 720x2160x2,
+    //   radix 8, 355 / 246.  Radix 8 of 1024 points takes the rows half as long again: 1024x2160x1
+    //   182 / 190, 1024x2160x3 472 / 514, 1024x2048x2 264 / 232, open 1024x1024x2 397 / 412,
+    //   1024x1024x3 624 / 653.  So it is left to columns of 512 values and more (1024x4096x1
+    //   264 / 222).  Where radix 8 does not pay, radix 4 follows (160, -, 222, 388, 613), over 512
+    //   values for one layer only (1024x2160x3 with 540 values 472 / 560, open 1024x1080x2
+    //   491 / 582).
     // one: the tensor is one that the kernel takes (z-offset blocks of six slots).  Any other
     // keeps the unsplit columns: over split ones its three kernels gained less in the columns
     // than the rows lost (a step, us, unequal layers: 256x2048x4 rows 27 / 27 a field against
@@ -522,13 +533,21 @@ struct Engine : EngineBase {
         subR = subRm = 1;
         colp = false;
         pcol = c->py;
+        bool no8 = false;   // radix 8 would fit, but does not pay
         for (int R = 8; R >= (c->open ? 2 : 1) && !colp && one && sizeof(T) == 8 && nl <= 4; R /= 2) {
             const int L = fy / R, rm = c->open ? R / 2 : R, ty = std::max(ty_def, rm);
             FFTPlan q;
             if (fy % R != 0 || L < 256 || !factorize(L, q)) continue;
+            if (nl == 4 && L != 256 && (c->open || L < 360 || L > 512)) continue;
             const size_t lc = sizeof(T) * 2 * LPN(3 * nl * L);
             const int th = lc > 56 * 1024 ? 512 : 256, e = pick_e(3 * nl, q, th);
             if (lc > 112 * 1024 || ty / 2 * c->fx > 4096 || ty > 16) continue;
+            if (R == 8 && ((ty / 2 * c->fx > 3072 && (c->open || L < 512)) ||
+                           (c->open && nl == 3 && L != 256 && L < 360))) {
+                no8 = true;
+                continue;
+            }
+            if (no8 && L > 512 && nl > 1) continue;
             if (pick_e(ty / 2, c->px, 256) < 0 || e < 0) continue;   // e: 14 at most, of 16
             subR = R;
             subRm = rm;

@@ -14,8 +14,8 @@ from tests.test_gpu_split_layout import context, convolution_error, load
 pytestmark = pytest.mark.gpu
 
 
-# 768, 540 and 810 rows of FFT: radix 4 would leave columns under 256
-@pytest.mark.parametrize("nx,ny,nl", [(32, 384, 3), (30, 270, 4), (20, 405, 3), (64, 384, 4)])
+# 768, 720, 810 and 1000 rows of FFT: radix 4 would leave columns under 256
+@pytest.mark.parametrize("nx,ny,nl", [(32, 384, 3), (30, 360, 3), (20, 405, 3), (64, 500, 3)])
 @pytest.mark.parametrize("tune", [{}, {"row_block": 2}, {"row_block": 4, "row_threads": 64},
                                   {"row_threads": 256, "col_radix": 4}, {"row_radix": 4, "col_radix": 8}])
 def test_radix_two_open(nx, ny, nl, tune):
@@ -33,7 +33,7 @@ def test_radix_two_open(nx, ny, nl, tune):
 
 
 @pytest.mark.parametrize("nx,ny,nl,open_,radix", [
-    (32, 384, 3, True, 2), (20, 405, 3, True, 2), (30, 540, 2, True, 4), (32, 1024, 3, True, 8), (45, 540, 4, False, 2),
+    (32, 384, 3, True, 2), (20, 405, 3, True, 2), (30, 540, 2, True, 4), (32, 1024, 3, True, 8), (45, 720, 4, False, 2),
     (32, 1024, 4, False, 4), (40, 2048, 4, False, 8)])
 def test_row_shapes_leave_the_values(nx, ny, nl, open_, radix):
     def run(tune):
@@ -55,7 +55,7 @@ def test_row_shapes_leave_the_values(nx, ny, nl, open_, radix):
         assert same(want, run(tune))
 
 
-@pytest.mark.parametrize("nx,ny,nl", [(24, 4096, 4), (1024, 2304, 1)])   # 98 KB a column kernel; 70 KB a row kernel
+@pytest.mark.parametrize("nx,ny,nl", [(24, 4096, 4), (2000, 1080, 2)])   # 98 KB a column kernel; 68 KB a row kernel
 def test_captured_batch_with_wide_lds(nx, ny, nl):
     med = media.make_media(nx, ny, dz=2e-7, n_lay=nl, seed=3, thermal=True, temperature=300.0)
 
@@ -92,4 +92,26 @@ def test_row_block_reads_what_is_launched(nx, ny, nl, open_, rows):
         assert x.get_tune("row_block") == max(v, rows)
         x.tune("row_block", x.get_tune("row_block"))
         assert x.get_tune("row_block") == max(v, rows)
+    x.close()
+
+
+# both sides of each limit of the layout's rule: 256 and 360 to 512 values a column of four
+# layers, 256 with open boundaries, other layers from 256 on; rows of 768 points with radix 8,
+# longer ones with columns of 512 values or with radix 4 and up to 512; the field is the
+# convolution's on each of the small ones
+@pytest.mark.parametrize("nx,ny,nl,open_,radix", [
+    (16, 1024, 4, False, 4), (16, 540, 4, False, 0), (16, 648, 4, False, 0), (16, 720, 4, False, 2), (16, 1080, 4, False, 0),
+    (16, 2160, 4, False, 0), (16, 3072, 4, False, 8), (16, 512, 4, True, 4), (16, 540, 4, True, 0), (16, 384, 4, True, 0),
+    (16, 360, 3, True, 2), (16, 720, 3, False, 2), (768, 2160, 1, False, 8), (800, 2160, 1, False, 4),
+    (768, 2160, 2, False, 8), (800, 2160, 2, False, 0), (800, 2048, 2, False, 4), (1024, 4096, 1, False, 8),
+    (2000, 1080, 2, False, 4), (450, 1080, 2, True, 0), (450, 1024, 2, True, 4), (384, 1080, 2, True, 8),
+    (1024, 1350, 2, False, 2), (64, 1080, 3, True, 0), (64, 1024, 3, True, 8)])
+def test_layout_rule(nx, ny, nl, open_, radix):
+    x, med = context(nx, ny, nl, 2e-7, open_)
+    N = x.build_tensor(num_images=0, return_real=nx * ny < 100000)
+    assert x.get_tune("col_split") == radix
+    if nx * ny < 100000:
+        load(x, med)
+        x.step(0, diag=False)
+        assert convolution_error(x, med, N) <= 1e-12
     x.close()
