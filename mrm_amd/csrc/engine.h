@@ -813,9 +813,11 @@ struct Engine : EngineBase {
         for (int k = 0; k < nl; k++) off[k + 1] = off[k] + L[k].ng;
         G = off[nl];
         // one lane per grain where 64 grains a wave fill the chip (256 CUs of 4 SIMDs, two
-        // waves each), else as many lanes as keep the waves of the chip busy; measured, us a
-        // stage: 523 704 grains 161 with 1 lane, 195 with 2, 253 with 4; 32 680 grains 34, 26,
-        // 23; 15 692 grains 15.9, 13.0, 11.0 and 10.7 with 8
+        // waves each), else as many lanes as keep the waves of the chip busy; two stages, us, of
+        // media without sources with 1 / 4 / 8 lanes: 251 052 grains 69 / 75 / 121, 132 500
+        // 49 / 47 / 71, 117 796 42 / 43 / 64, 62 764 34 / 27 / 40, 24 872 32 / 20 / 26, 23 096
+        // 32 / 20 / 22, 15 712 31 / 18 / 19; under a moving spot 523 704 grains 161 a stage with 1,
+        // 253 with 4
         if (!lpg_set) lpg = G >= 131072 ? 1 : G >= 24576 ? 4 : 8;
         Ctot = 0;
         for (int k = 0; k < nl; k++) Ctot += L[k].ncell;
