@@ -402,8 +402,8 @@ int mrmg_tune(mrmg_ctx *ctx, const char *key, int value);
  * only through ko - ks: equal thicknesses and spacings, no magnetic images above or
  * below), 0 when they are the n_lay^2 layer-pair blocks; or "col_split": where the column
  * FFTs, the product and the inverse run as one kernel between row kernels that take a radix
- * of the column transform (FP64, grids for the split path, up to 4 layers, z-offset tensor
- * of 6 slots), that radix (1: none of it), else 0. */
+ * of the column transform (FP64, those grids for the split path that gain by it, up to 4
+ * layers, z-offset tensor of 6 slots), that radix (1: none of it), else 0. */
 int mrmg_get_tune(mrmg_ctx *ctx, const char *key, int *value);
 /* Copies up to max entries; *n receives the number of kernel classes. */
 int mrmg_kernel_stats(mrmg_ctx *ctx, mrmg_kstat *out, int max, int *n);

@@ -337,7 +337,7 @@ struct Engine : EngineBase {
     // the split of the column transform (RowSplit): its radix, the media rows of a group; the
     // one-kernel column path (colprod.hip) and its launch shape
     int subR = 1, subRm = 1, colp_threads = 256, ty_def = 8;   // ty_def: TYr before any row_block
-    bool colp = false, one_fit = true;                         // one_fit: choose_split's argument
+    bool colp = false, one_fit = true, fit_ok = true;          // one_fit: choose_split's argument
     size_t lds_colp = 0;
     DBuf<C2<T>> tws;
     // FFT plans of the step's row and column transforms and their largest radix
@@ -589,8 +589,8 @@ struct Engine : EngineBase {
     int fit_split(bool toeplitz)
     {
         const bool one = (toeplitz || c->nl == 1) && nslot == 6;   // one layer: one block either way
-        if (fused_ok || sizeof(T) != 8 || c->nl > 4 || one == one_fit) return MRMG_OK;
-        tensor_ok = false;
+        if (fused_ok || sizeof(T) != 8 || c->nl > 4 || (one == one_fit && fit_ok)) return MRMG_OK;
+        tensor_ok = fit_ok = false;   // fit_ok: a call that failed half way is done again by the next
         HIPCHK(hipStreamSynchronize(c->stream));
         const bool def = row_threads == row_def;
         RCHK(choose_split(one));
@@ -599,6 +599,7 @@ struct Engine : EngineBase {
         RCHK(shapes());
         RCHK(lds_attr());
         one_fit = one;
+        fit_ok = true;
         return MRMG_OK;
     }
     // the columns as laid out: vnx() per plane, of vL() values
